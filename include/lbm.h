@@ -208,10 +208,12 @@ int lbm_set_force(lbm_ctx* ctx, const float in[3]);
 int lbm_get_force(lbm_ctx* ctx, float out[3]);
 
 /* ------------------------------------------------------------ stepping */
-/* n fused steps.  Standard mode: BGK pull collide+stream (D2Q9 lattices
- * with 16-bit storage larger than the Infinity Cache are updated 4 or 2
- * nodes per thread; the environment variable LBM_GROUP_STEP=0 / 1 turns
- * that off / on for any size -- the results are the same bytes).
+/* n fused steps.  Standard mode: BGK pull collide+stream (large D2Q9
+ * lattices take up to four steps in one pass over memory; one step of a
+ * D2Q9 lattice with 16-bit storage larger than the Infinity Cache updates 4
+ * or 2 nodes per thread; the environment variable LBM_GROUP_STEP=0 / 1 asks
+ * for one step at a time and turns the latter off / on for any size -- the
+ * results are the same bytes).
  * Reference mode: Lattice::simulateLattice (Lattice.cpp:222-226), stream
  * then collide. */
 int lbm_step(lbm_ctx* ctx, int n);

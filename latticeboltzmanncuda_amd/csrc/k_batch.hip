@@ -58,6 +58,21 @@ __global__ void __launch_bounds__(kMaxBatchBlock)
   }
 }
 
+// K steps of every D2Q9 lattice (sweep_unit), one unit per wavefront.
+template <int S, int K>
+__global__ void __launch_bounds__(64 * kSweepWaves)
+    k_batch_sweep(const BatchLattice* __restrict__ lats, const BatchTile* __restrict__ units,
+                  const uint32_t* __restrict__ nunits, int parity) {
+  using T = typename Store<S>::T;
+  const uint32_t w =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * kSweepWaves + (threadIdx.x >> 6));
+  if (w >= *nunits) return;
+  const BatchTile unit = units[w];
+  const BatchLattice& L = lats[unit.lat];
+  const int cur = (L.off + parity) & 1;
+  sweep_unit<S, K>(L.g, L.sweep, (const T*)L.f[cur], (T*)L.f[cur ^ 1], L.mask, L.p, unit.first);
+}
+
 __device__ __forceinline__ double block_sum(double v, double* red) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -186,6 +201,19 @@ int launch_batch_step(int storage, int cls, bool nt, int block, int grid,
     rc = launch_step_q<Tag::Q, Tag::S>(nt, block, grid, lats, tiles, ntiles, parity, s);
   });
   return drc ? drc : rc;
+}
+
+int launch_batch_sweep(int storage, int k, int grid, const BatchLattice* lats,
+                       const BatchTile* units, const uint32_t* nunits, int parity, hipStream_t s) {
+  if (grid <= 0) return fail(LBM_ERR_INVALID, "batch grid must be positive");
+  const int drc = dispatch_sweep(storage, k, [&](auto tag, auto steps) {
+    constexpr int S = decltype(tag)::S, K = decltype(steps)::value;
+    hipLaunchKernelGGL((k_batch_sweep<S, K>), dim3((unsigned)grid), dim3(64 * kSweepWaves), 0, s,
+                       lats, units, nunits, parity);
+  });
+  if (drc) return drc;
+  LBM_HIP(hipGetLastError());
+  return LBM_OK;
 }
 
 int launch_batch_residual(int storage, const BatchLattice* lats,

@@ -21,6 +21,7 @@
 #include "lbm_layout.h"
 #include "lbm_step_node.h"
 #include "lbm_store.h"
+#include "lbm_sweep.h"
 
 namespace lbm {
 namespace {
@@ -77,6 +78,18 @@ __global__ void __launch_bounds__(kBlock)
   const uint32_t n0 = (blk * kBlock + threadIdx.x) * (uint32_t)NV;
   if (n0 >= g.n) return;  // the rows of active groups are whole
   std_group_step<Q, S, NV, LID, NT>(g, A, B, mask, cls, p, n0);
+}
+
+// K steps of a D2Q9 lattice in one pass (sweep_unit), one unit per wavefront.
+template <int S, int K>
+__global__ void __launch_bounds__(kBlock)
+    k_std_sweep(Grid g, SweepPlan pl, const typename Store<S>::T* __restrict__ A,
+                typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
+                StdParams p) {
+  const uint32_t u =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6));
+  if (u >= pl.units) return;
+  sweep_unit<S, K>(g, pl, A, B, mask, p, u);
 }
 
 template <int Q>
@@ -390,6 +403,29 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
     else
       hipLaunchKernelGGL((k_std_step<Tag::Q, Tag::S, false, false>), grid, block, 0, s, g, a, b,
                          mask, cls, p, r);
+  });
+  if (drc) return drc;
+  LBM_HIP(hipGetLastError());
+  return LBM_OK;
+}
+
+bool std_sweeps(int q, int storage, const Grid& g) {
+  const char* env = std::getenv("LBM_GROUP_STEP");  // asks for steps one at a time
+  if (q != 9 || (env && (env[0] == '0' || env[0] == '1'))) return false;
+  // 16-bit lattices that fit the Infinity Cache are as fast one step at a
+  // time (2900 x 1700: 24.2-30.5 against 24.7-28.9 us), larger ones are not
+  return storage_bytes(storage) == 2 ? streaming_stores(2 * population_elems(q, g.n) * 2)
+                                     : g.n >= kSweepMinNodes;
+}
+
+int launch_std_sweep(int k, int storage, const Grid& g, const SweepPlan& pl, const void* A,
+                     void* B, const uint32_t* mask, const StdParams& p, hipStream_t s) {
+  const dim3 grid((pl.units + kBlock / 64 - 1) / (kBlock / 64));
+  const int drc = dispatch_sweep(storage, k, [&](auto tag, auto steps) {
+    constexpr int S = decltype(tag)::S, K = decltype(steps)::value;
+    using T = typename Store<S>::T;
+    hipLaunchKernelGGL((k_std_sweep<S, K>), grid, dim3(kBlock), 0, s, g, pl, (const T*)A, (T*)B,
+                       mask, p);
   });
   if (drc) return drc;
   LBM_HIP(hipGetLastError());

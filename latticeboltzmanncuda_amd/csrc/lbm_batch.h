@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "lbm_internal.h"
+#include "lbm_sweep.h"
 
 namespace lbm {
 
@@ -32,6 +33,7 @@ struct BatchLattice {
   int32_t off;
   float* u_prev;           // velocity snapshot for residuals (3 x N)
   uint32_t res_first;      // first residual chunk of this lattice
+  SweepPlan sweep;         // D2Q9: how its sweeps are cut
 };
 
 struct BatchTile {
@@ -58,6 +60,11 @@ inline int class_q(int c) { return c == 0 ? 9 : (c == 1 ? 19 : 27); }
 int launch_batch_step(int storage, int cls, bool nt, int block, int grid,
                       const BatchLattice* lats, const BatchTile* tiles,
                       const uint32_t* ntiles, int parity, hipStream_t s);
+// k steps (2 to 4) of the D2Q9 lattices, whose sweep units are listed in
+// `units` (lattice, unit); grid: workgroups of kSweepWaves wavefronts.
+constexpr int kSweepWaves = 4;
+int launch_batch_sweep(int storage, int k, int grid, const BatchLattice* lats,
+                       const BatchTile* units, const uint32_t* nunits, int parity, hipStream_t s);
 int launch_batch_residual(int storage, const BatchLattice* lats,
                           const BatchTile* chunks, uint32_t nchunks,
                           double* partials, hipStream_t s);
@@ -83,7 +90,11 @@ struct lbm_batch {
   uint32_t lats_cap = 0;
   lbm::BatchTile* d_tiles[lbm::kBatchClasses] = {};
   uint32_t tiles_cap[lbm::kBatchClasses] = {};
-  uint32_t* d_ntiles = nullptr;  // tiles per class (device copy)
+  uint32_t* d_ntiles = nullptr;  // tiles per class, sweep units (device copy)
+  // D2Q9 members' sweep units (lattice, unit); none where the sweep is not
+  // used for them
+  lbm::BatchTile* d_units = nullptr;
+  uint32_t units_cap = 0, nunits = 0;
   lbm::BatchTile* d_chunks = nullptr;  // residual chunks
   uint32_t chunks_cap = 0;
   double* d_partials = nullptr;        // 2 per residual chunk
@@ -114,4 +125,6 @@ struct lbm_batch {
   // a class that was empty)
   void* graph_tables[lbm::kBatchClasses] = {};
   int graph_grids[lbm::kBatchClasses] = {};
+  const void* graph_units = nullptr;  // sweep units and grid, likewise
+  int graph_sweep_grid = 0;
 };

@@ -21,6 +21,7 @@
 #include "lbm_lattice.h"
 #include "lbm_layout.h"
 #include "lbm_store.h"
+#include "lbm_sweep.h"
 
 namespace lbm {
 
@@ -516,13 +517,23 @@ int rebuild_special(lbm_ctx* c) {
 
 int step_standard(lbm_ctx* c, int n) {
   const StdParams p = make_std_params(c->cfg);
-  for (int s = 0; s < n; ++s) {
-    int rc = launch_std_step(c->q, device_storage(c->cfg.mode, c->cfg.storage), c->grid, c->f[c->cur],
-                             c->f[c->cur ^ 1], c->mask, c->cls, p,
-                             (int)(c->steps_done & 1), c->stream);
+  const int storage = device_storage(c->cfg.mode, c->cfg.storage);
+  const bool sweeps = n > 1 && std_sweeps(c->q, storage, c->grid);
+  const SweepPlan plan =
+      sweeps ? sweep_plan(c->grid, sweep_chunk_rows(
+                                       1, [&](size_t) -> const Grid& { return c->grid; }, storage))
+             : SweepPlan{};
+  const int passes = sweeps ? sweep_passes(n, false) : n;
+  for (int s = 0, left = n; s < passes; ++s) {
+    const int k = (left + (passes - s) - 1) / (passes - s);
+    int rc = k > 1 ? launch_std_sweep(k, storage, c->grid, plan, c->f[c->cur], c->f[c->cur ^ 1],
+                                      c->mask, p, c->stream)
+                   : launch_std_step(c->q, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1],
+                                     c->mask, c->cls, p, (int)(c->steps_done & 1), c->stream);
     if (rc) return rc;
     c->cur ^= 1;
-    ++c->steps_done;
+    c->steps_done += k;
+    left -= k;
   }
   return LBM_OK;
 }

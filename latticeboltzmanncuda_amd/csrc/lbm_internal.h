@@ -135,6 +135,12 @@ int api_exception() noexcept;
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
                     const uint32_t* mask, const uint32_t* cls,
                     const StdParams& p, int rev, hipStream_t s);
+// Whether several steps of a lattice are taken in one pass over memory
+// (launch_std_sweep, k of 2 to 4 steps; large D2Q9 lattices).
+struct SweepPlan;
+bool std_sweeps(int q, int storage, const Grid& g);
+int launch_std_sweep(int k, int storage, const Grid& g, const SweepPlan& pl, const void* A,
+                     void* B, const uint32_t* mask, const StdParams& p, hipStream_t s);
 int launch_build_mask(int q, const Grid& g, const uint8_t* solid,
                       const int periodic[3], int lid_face, uint32_t* mask,
                       uint32_t* cls, hipStream_t s);

@@ -291,6 +291,27 @@ __device__ __forceinline__ void std_gather(const Grid& g,
   }
 }
 
+// s * b + c rounded once to FP16 (v_fma_mixlo_f16; s is uniform).  Written
+// out because the compiler folds the conversion into the fma in some
+// surroundings and not in others, which rounds twice: every kernel has to
+// round alike.
+__device__ __forceinline__ _Float16 fma_to_half(float s, float b, float c) {
+  uint32_t r;
+  __asm__("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(r) : "s"(s), "v"(b), "v"(c));
+  return __builtin_bit_cast(_Float16, (uint16_t)r);
+}
+
+// an output of std_relax in the stored type (already there, or still to be
+// rounded)
+template <int S>
+__device__ __forceinline__ typename Store<S>::T round_out(typename Store<S>::C o) {
+  return Store<S>::round_u(o);
+}
+template <int S>
+__device__ __forceinline__ _Float16 round_out(_Float16 o) {
+  return o;
+}
+
 template <bool B>
 struct Forced {
   static constexpr bool value = B;
@@ -342,6 +363,13 @@ __device__ __forceinline__ void std_relax(const StepCoef<typename Store<S>::C>& 
     const C d = k16 ? fmadd(wu, fmadd(t, rho, rs), -gv[i])
                 : kSh ? fmadd(wu, fmadd(rs, t, t + rs), -gv[i])
                       : (w * rs) * t - gv[i];
+    if constexpr (S == LBM_STORE_F16 && !FORCED) {
+      // the last fma rounds once, to FP16 (fma_to_half)
+      _Float16 o = fma_to_half(k.omega, d, gv[i]);
+      if (SOLID) o = solid ? (_Float16)0.0f : o;
+      emit(Forced<FORCED>{}, i, o);
+      continue;
+    }
     C out = fmadd(k.omega, d, gv[i]);
     if (FORCED) {
       // Guo source (1 - omega/2) w (3 (e.F - u.F) + 9 (e.u)(e.F)), added
@@ -361,7 +389,11 @@ __device__ __forceinline__ void std_relax(const StepCoef<typename Store<S>::C>& 
 // stored form and stored units, gv[i] (f_i, or f_i - w_i for shifted
 // storage), its link mask m and solid flag; emit receives the outputs (see
 // std_relax).
-template <int Q, int S, bool LID, class Emit>
+// FORCE: whether the lattice has a body force, known to the caller (0 / 1)
+// or read from the lattice's constants (2).  SOLID: whether the wavefront
+// may hold solid nodes whose outputs matter (0: no, 1: yes, 2: found out
+// here).
+template <int Q, int S, bool LID, int FORCE = 2, int SOLID = 2, class Emit>
 __device__ __forceinline__ void std_collide_node(const StdParams& p,
                                                  typename Store<S>::C (&gv)[Q], uint32_t m,
                                                  bool solid, Emit&& emit) {
@@ -420,10 +452,11 @@ __device__ __forceinline__ void std_collide_node(const StdParams& p,
   // lattices' batch kernels registers (their eight waves per SIMD then
   // spill to memory)
   constexpr bool kSkipSolid = Q == 9 && sizeof(typename St::T) == 2;
-  const bool any_solid = !kSkipSolid || __builtin_amdgcn_ballot_w64(solid) != 0;
+  const bool any_solid =
+      SOLID == 2 ? !kSkipSolid || __builtin_amdgcn_ballot_w64(solid) != 0 : SOLID == 1;
   // D2Q9 has no z velocity (its z force is 0: lbm_create checks)
   constexpr bool k2D = L::D == 2;
-  if (k.forced) {
+  if (FORCE == 2 ? k.forced != 0 : FORCE == 1) {
     const C ux = (jx + k.half_force[0]) * ir;
     const C uy = (jy + k.half_force[1]) * ir;
     const C uz = k2D ? (C)0 : (jz + k.half_force[2]) * ir;
@@ -458,7 +491,7 @@ __device__ __forceinline__ void std_collide(const StdParams& p,
   using T = typename St::T;
   T* const out0 = B + ld.own;
   const auto rsrc = buffer_rsrc(B, ld.pop_bytes);
-  std_collide_node<Q, S, LID>(p, gv, ld.m, ld.solid, [&](auto forced, int i, C out) {
+  std_collide_node<Q, S, LID>(p, gv, ld.m, ld.solid, [&](auto forced, int i, auto out) {
     // a body force moves 16-bit populations by less than their rounding
     // step: those lattices round stochastically (no effect at full
     // precision)
@@ -466,7 +499,7 @@ __device__ __forceinline__ void std_collide(const StdParams& p,
     if constexpr (decltype(forced)::value)
       v = St::round_sr_u(out, sr_key(St::kShifted ? sr_node_hash(ld.own) : 0u, i));
     else
-      v = St::round_u(out);
+      v = round_out<S>(out);
     if constexpr (sizeof(T) == 2)
       bstore16<NT>(rsrc, 2u * ld.own + (uint32_t)(i * kTile * 2), v);
     else if (NT)
@@ -670,11 +703,11 @@ __device__ __forceinline__ void std_group_step(
     C gv[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i) gv[i] = St::cvt_u(V[i][k]);
-    std_collide_node<Q, S, LID>(p, gv, m[k], solid[k], [&](auto forced, int i, C out) {
+    std_collide_node<Q, S, LID>(p, gv, m[k], solid[k], [&](auto forced, int i, auto out) {
       if constexpr (decltype(forced)::value)
         V[i][k] = St::round_sr_u(out, sr_key(St::kShifted ? sr_node_hash(own + k) : 0u, i));
       else
-        V[i][k] = St::round_u(out);
+        V[i][k] = round_out<S>(out);
     });
   }
   T* const out0 = B + own;
