@@ -27,7 +27,7 @@ template <int Q, int S>
 __global__ void __launch_bounds__(kBlock)
     k_points_in(Grid g, const lbm_lattice_point* __restrict__ pts,
                 typename Store<S>::T* __restrict__ f,
-                uint8_t* __restrict__ flags) {
+                uint8_t* __restrict__ flags, int* __restrict__ changed) {
   using L = Lat<Q>;
   using St = Store<S>;
   const uint32_t n = blockIdx.x * kBlock + threadIdx.x;
@@ -39,9 +39,14 @@ __global__ void __launch_bounds__(kBlock)
     if (St::kShifted) v -= (float)L::W[i];
     St::store(f + pidx<Q>(n, i), (typename St::C)v);
   }
-  if (flags)
-    flags[n] = (uint8_t)((p->isInternal ? LBM_FLAG_INTERNAL : 0u) |
-                         (p->isReflected ? LBM_FLAG_REFLECTED : 0u));
+  if (flags) {
+    const uint8_t fl = (uint8_t)((p->isInternal ? LBM_FLAG_INTERNAL : 0u) |
+                                 (p->isReflected ? LBM_FLAG_REFLECTED : 0u));
+    if (flags[n] != fl) {
+      flags[n] = fl;
+      *changed = 1;  // any thread's store says the same
+    }
+  }
 }
 
 template <int Q, int S>
@@ -128,12 +133,12 @@ int launch_copy_stream(const void* src, void* dst, uint64_t bytes, hipStream_t s
 
 int launch_points_in(int q, int storage, const Grid& g,
                      const lbm_lattice_point* pts, void* f, uint8_t* flags,
-                     hipStream_t s) {
+                     int* changed, hipStream_t s) {
   const int drc = dispatch_qs(q, storage, [&](auto tag) {
     using Tag = decltype(tag);
     using T = typename Store<Tag::S>::T;
     hipLaunchKernelGGL((k_points_in<Tag::Q, Tag::S>), dim3(blocks_for(g.n)),
-                       dim3(kBlock), 0, s, g, pts, (T*)f, flags);
+                       dim3(kBlock), 0, s, g, pts, (T*)f, flags, changed);
   });
   if (drc) return drc;
   LBM_HIP(hipGetLastError());

@@ -286,231 +286,10 @@ int validate_config(const lbm_config* cfg) {
   return LBM_OK;
 }
 
-// Tables of the fused reference step.  Every slot s (1..80) of a
-// reflecting node x with direction d (1..26) whose target t = x + e_d lies
-// in the box becomes an entry of group (t, d); a group's entries keep
-// ascending s, the order in which the staged reflection pass adds them, and
-// groups are ordered by (t, d).  Targets must not be flagged: the staged
-// pass would otherwise race between adding to a target and zeroing it.
-int rebuild_receivers(lbm_ctx* c, const std::vector<int32_t>& rec_of) {
-  const Grid& g = c->grid;
-  const int64_t N = g.n;
-  const size_t words = (size_t)((N + 15) / 16);
-  const size_t ng = (size_t)std::max<int64_t>(c->ref_ngrp, 1), ne = (size_t)std::max<int64_t>(c->ref_nent, 1);
-  dev_free(c, (void**)&c->ref_cls, sizeof(uint32_t) * words);
-  const size_t kwords = (size_t)((N + 64 * 32 - 1) / (64 * 32));
-  dev_free(c, (void**)&c->ref_keep, sizeof(uint32_t) * kwords);
-  dev_free(c, (void**)&c->ref_inmask, sizeof(uint32_t) * (size_t)N);
-  dev_free(c, (void**)&c->ref_rxbase, sizeof(int32_t) * (size_t)N);
-  dev_free(c, (void**)&c->ref_gsrc, sizeof(uint32_t) * ng);
-  dev_free(c, (void**)&c->ref_gbeg, sizeof(uint32_t) * ng);
-  dev_free(c, (void**)&c->ref_gid, sizeof(uint32_t) * ng);
-  dev_free(c, (void**)&c->ref_gsum, sizeof(float) * ng);
-  dev_free(c, (void**)&c->ref_eidx, sizeof(uint32_t) * ne);
-  dev_free(c, (void**)&c->ref_ew, sizeof(float) * ne);
-  dev_free(c, (void**)&c->ref_es, sizeof(uint8_t) * ne);
-  dev_free(c, (void**)&c->ref_partials, sizeof(float) * 3 * (size_t)std::max(c->ref_partials_cap, 1));
-  c->ref_ngrp = c->ref_nent = 0;
-  c->ref_partials_cap = 0;
-  c->ref_geom = c->nspecial > 0;
-  if (!c->ref_geom) return LBM_OK;
-
-  struct Link {
-    uint32_t t;   // receiving node
-    uint8_t d;    // direction of the reflected population
-    uint8_t s;    // slot of the reflecting node's record
-    int32_t r;    // record
-  };
-  const int64_t plane = (int64_t)g.ny * g.nz;
-  auto at = [&](int64_t x, int64_t y, int64_t z) { return z + (int64_t)g.nz * (y + (int64_t)g.ny * x); };
-  std::vector<Link> links;
-  std::vector<uint32_t> cls(words, 0u);
-  for (int64_t n = 0; n < N; ++n) {
-    const uint8_t fl = c->host_flags[n];
-    if (fl & LBM_FLAG_INTERNAL) cls[n >> 4] |= 2u << (2 * (n & 15));
-    const int32_t r = c->nrec > 0 ? rec_of[n] : -1;
-    if (!(fl & LBM_FLAG_REFLECTED) || r < 0) continue;
-    const int64_t x = n / plane, y = (n % plane) / g.nz, z = n % g.nz;
-    const uint32_t* w = c->host_rec_dirs.data() + 14 * (size_t)r;
-    for (int s = 1; s < 81; ++s) {
-      const int d = (int)((w[s / 6] >> (5 * (s % 6))) & 0x1Fu);
-      if (d == 0 || d > 26) continue;
-      const int64_t tx = x + Lat<27>::E[d][0], ty = y + Lat<27>::E[d][1], tz = z + Lat<27>::E[d][2];
-      if (tx < 0 || ty < 0 || tz < 0 || tx >= g.nx || ty >= g.ny || tz >= g.nz) continue;
-      const int64_t t = at(tx, ty, tz);
-      if (c->host_flags[t])
-        return fail(LBM_ERR_INVALID, "reflection target " + std::to_string(t) +
-                                         " is a flagged node (targets must be fluid)");
-      links.push_back({(uint32_t)t, (uint8_t)d, (uint8_t)s, r});
-    }
-  }
-  std::stable_sort(links.begin(), links.end(), [](const Link& a, const Link& b) {
-    return a.t != b.t ? a.t < b.t : (a.d != b.d ? a.d < b.d : a.s < b.s);
-  });
-  std::vector<uint32_t> inmask((size_t)N, 0u), gsrc, gbeg, eidx;
-  std::vector<int32_t> base((size_t)N, -1);
-  std::vector<float> ew;
-  std::vector<uint8_t> es;
-  for (size_t i = 0; i < links.size();) {
-    const uint32_t t = links[i].t;
-    base[t] = (int32_t)gsrc.size();
-    cls[t >> 4] |= 1u << (2 * (t & 15));
-    const int64_t tx = t / plane, ty = (t % plane) / g.nz, tz = t % g.nz;
-    while (i < links.size() && links[i].t == t) {
-      const int d = links[i].d;
-      inmask[t] |= 1u << d;
-      // the reflecting node x = t - e_d (inside the box: it holds a record)
-      const int64_t xx = tx - Lat<27>::E[d][0], xy = ty - Lat<27>::E[d][1], xz = tz - Lat<27>::E[d][2];
-      gsrc.push_back(pidx<27>((uint32_t)at(xx, xy, xz), d));
-      gbeg.push_back((uint32_t)eidx.size());
-      for (; i < links.size() && links[i].t == t && links[i].d == d; ++i) {
-        const int s = links[i].s, k = s / 3;
-        // x's streamed value of direction k: A_k(x - e_k), 0 outside
-        const int64_t sx = xx - Lat<27>::E[k][0], sy = xy - Lat<27>::E[k][1], sz = xz - Lat<27>::E[k][2];
-        const bool in = sx >= 0 && sy >= 0 && sz >= 0 && sx < g.nx && sy < g.ny && sz < g.nz;
-        eidx.push_back(in ? pidx<27>((uint32_t)at(sx, sy, sz), k) : ~0u);
-        ew.push_back(c->host_rec_w[81 * (size_t)links[i].r + (size_t)s]);
-        es.push_back((uint8_t)s);
-      }
-    }
-  }
-  if (eidx.size() >= (1ull << 31)) return fail(LBM_ERR_UNSUPPORTED, "too many reflected links");
-  // The gather's threads take the groups by reflecting node x, then
-  // direction (gsrc = pidx(x, d) gives both): the groups of one x read the
-  // same neighbours of x (up to three slots share an incoming direction),
-  // so a wavefront touches fewer cache lines than in receiver order (on
-  // the 128^3 angled cube 193 k lines over all wavefronts against 295 k).
-  // Each thread writes its sum to its group's slot; the tables follow the
-  // thread order.
-  const size_t ngs = gsrc.size();
-  std::vector<uint32_t> gid(ngs);
-  for (size_t q = 0; q < ngs; ++q) gid[q] = (uint32_t)q;
-  auto xd = [&](uint32_t q) {
-    const uint32_t e = gsrc[q];
-    const uint64_t x = (uint64_t)(e / (27u * kTile)) * kTile + e % kTile;
-    return x * 32u + (e / kTile) % 27u;
-  };
-  std::stable_sort(gid.begin(), gid.end(), [&](uint32_t a, uint32_t b) { return xd(a) < xd(b); });
-  {
-    std::vector<uint32_t> tsrc(ngs), tbeg(ngs), te(eidx.size());
-    std::vector<float> tw(ew.size());
-    std::vector<uint8_t> ts(es.size());
-    size_t pos = 0;
-    for (size_t i = 0; i < ngs; ++i) {
-      const uint32_t q = gid[i];
-      const size_t b = gbeg[q], e = q + 1 < ngs ? gbeg[q + 1] : eidx.size();
-      tsrc[i] = gsrc[q];
-      tbeg[i] = (uint32_t)pos;
-      for (size_t k = b; k < e; ++k, ++pos) {
-        te[pos] = eidx[k];
-        tw[pos] = ew[k];
-        ts[pos] = es[k];
-      }
-    }
-    gsrc.swap(tsrc);
-    gbeg.swap(tbeg);
-    eidx.swap(te);
-    ew.swap(tw);
-    es.swap(ts);
-  }
-  c->ref_ngrp = (int64_t)gsrc.size();
-  c->ref_nent = (int64_t)eidx.size();
-  c->ref_partials_cap = ref_gather_partials(c->ref_ngrp);
-  const size_t ng2 = std::max<size_t>(gsrc.size(), 1), ne2 = std::max<size_t>(eidx.size(), 1);
-  int rc;
-  // tiles within two nodes of a reflecting node: the gather reads those
-  // within one, and the fused pass all of them (on the 128^3 angled cube a
-  // reach of 2 to 8 nodes gave 85.0-85.1 us per step, 1 node 85.6, 16
-  // nodes 85.6-85.7: the caches start to lose them)
-  constexpr int kKeepReach = 2;
-  std::vector<uint32_t> keep(kwords, 0u);
-  for (int64_t n = 0; n < N; ++n) {
-    if (!(c->host_flags[n] & LBM_FLAG_REFLECTED) || (c->nrec > 0 ? rec_of[n] : -1) < 0) continue;
-    const int64_t x = n / plane, y = (n % plane) / g.nz, z = n % g.nz;
-    for (int dx = -kKeepReach; dx <= kKeepReach; ++dx)
-      for (int dy = -kKeepReach; dy <= kKeepReach; ++dy)
-        for (int dz = -kKeepReach; dz <= kKeepReach; ++dz) {
-          const int64_t a = x + dx, b = y + dy, cz = z + dz;
-          if (a < 0 || b < 0 || cz < 0 || a >= g.nx || b >= g.ny || cz >= g.nz) continue;
-          const uint64_t tile = (uint64_t)at(a, b, cz) / 64u;
-          keep[tile >> 5] |= 1u << (tile & 31u);
-        }
-  }
-  if ((rc = dev_alloc(c, (void**)&c->ref_cls, sizeof(uint32_t) * words, "hipMalloc(ref classes)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_keep, sizeof(uint32_t) * kwords, "hipMalloc(ref tiles)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_inmask, sizeof(uint32_t) * (size_t)N, "hipMalloc(ref in-masks)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_rxbase, sizeof(int32_t) * (size_t)N, "hipMalloc(ref receivers)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_gsrc, sizeof(uint32_t) * ng2, "hipMalloc(ref groups)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_gbeg, sizeof(uint32_t) * ng2, "hipMalloc(ref groups)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_gid, sizeof(uint32_t) * ng2, "hipMalloc(ref groups)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_gsum, sizeof(float) * ng2, "hipMalloc(ref group sums)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_eidx, sizeof(uint32_t) * ne2, "hipMalloc(ref entries)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_ew, sizeof(float) * ne2, "hipMalloc(ref weights)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_es, sizeof(uint8_t) * ne2, "hipMalloc(ref slots)")) ||
-      (rc = dev_alloc(c, (void**)&c->ref_partials, sizeof(float) * 3 * (size_t)std::max(c->ref_partials_cap, 1),
-                      "hipMalloc(ref force partials)")))
-    return rc;
-  if ((rc = h2d(c, c->ref_cls, cls.data(), sizeof(uint32_t) * words)) ||
-      (rc = h2d(c, c->ref_keep, keep.data(), sizeof(uint32_t) * kwords)) ||
-      (rc = h2d(c, c->ref_inmask, inmask.data(), sizeof(uint32_t) * (size_t)N)) ||
-      (rc = h2d(c, c->ref_rxbase, base.data(), sizeof(int32_t) * (size_t)N)))
-    return rc;
-  if (!gsrc.empty() &&
-      ((rc = h2d(c, c->ref_gsrc, gsrc.data(), sizeof(uint32_t) * gsrc.size())) ||
-       (rc = h2d(c, c->ref_gbeg, gbeg.data(), sizeof(uint32_t) * gbeg.size())) ||
-       (rc = h2d(c, c->ref_gid, gid.data(), sizeof(uint32_t) * gid.size())) ||
-       (rc = h2d(c, c->ref_eidx, eidx.data(), sizeof(uint32_t) * eidx.size())) ||
-       (rc = h2d(c, c->ref_ew, ew.data(), sizeof(float) * ew.size())) ||
-       (rc = h2d(c, c->ref_es, es.data(), sizeof(uint8_t) * es.size()))))
-    return rc;
-  return LBM_OK;
-}
-
-// Nodes with a nonzero flag byte and their reflection record (or -1).
+// The geometry tables, rebuilt after a change of flags or records.
 int rebuild_special(lbm_ctx* c) {
   if (!c->special_dirty) return LBM_OK;
-  const int64_t N = c->grid.n;
-  std::vector<int32_t> rec_of;
-  if (c->nrec > 0) {
-    rec_of.assign((size_t)N, -1);
-    for (int32_t r = 0; r < c->nrec; ++r) {
-      const int32_t node = c->host_rec_node[r];
-      if (rec_of[node] >= 0)
-        return fail(LBM_ERR_INVALID, "two reflection records for node " +
-                                         std::to_string(node));
-      rec_of[node] = r;
-    }
-  }
-  std::vector<int32_t> sp, sr;
-  for (int64_t n = 0; n < N; ++n) {
-    const uint8_t fl = c->host_flags[n];
-    if (!fl) continue;
-    const int32_t r = c->nrec > 0 ? rec_of[n] : -1;
-    if ((fl & LBM_FLAG_REFLECTED) && r >= 0 && !(fl & LBM_FLAG_INTERNAL))
-      return fail(LBM_ERR_INVALID,
-                  "reflecting node " + std::to_string(n) +
-                      " is not internal (reflection runs in place and needs "
-                      "reflecting nodes inside the obstacle)");
-    sp.push_back((int32_t)n);
-    sr.push_back(r);
-  }
-  dev_free(c, (void**)&c->special, sizeof(int32_t) * (size_t)std::max(c->nspecial, 1));
-  dev_free(c, (void**)&c->special_rec, sizeof(int32_t) * (size_t)std::max(c->nspecial, 1));
-  dev_free(c, (void**)&c->force_partials, sizeof(float) * 3 * (size_t)std::max(c->force_partials_cap, 1));
-  c->nspecial = (int32_t)sp.size();
-  c->force_partials_cap = std::max(1, ref_reflect_blocks(c->nspecial));
-  int rc;
-  if ((rc = dev_alloc(c, (void**)&c->special, sizeof(int32_t) * std::max<size_t>(sp.size(), 1), "hipMalloc(special)")))
-    return rc;
-  if ((rc = dev_alloc(c, (void**)&c->special_rec, sizeof(int32_t) * std::max<size_t>(sr.size(), 1), "hipMalloc(special_rec)")))
-    return rc;
-  if ((rc = dev_alloc(c, (void**)&c->force_partials, sizeof(float) * 3 * (size_t)c->force_partials_cap, "hipMalloc(force partials)")))
-    return rc;
-  if (!sp.empty()) {
-    if ((rc = h2d(c, c->special, sp.data(), sizeof(int32_t) * sp.size()))) return rc;
-    if ((rc = h2d(c, c->special_rec, sr.data(), sizeof(int32_t) * sr.size()))) return rc;
-  }
-  if ((rc = rebuild_receivers(c, rec_of))) return rc;
+  if (int rc = build_receivers(c)) return rc;
   c->special_dirty = false;
   return LBM_OK;
 }
@@ -712,7 +491,6 @@ int lbm_create(const lbm_config* cfg, void* stream, lbm_ctx** out) {
       return bail(rc);
     if ((e = hipMemsetAsync(c->flags, 0, g.n, c->stream)) != hipSuccess)
       return bail(hip_fail(e, "hipMemsetAsync(flags)"));
-    c->host_flags.assign(g.n, 0);
   }
   if ((rc = sync(c))) return bail(rc);
   *out = c;
@@ -724,13 +502,8 @@ int lbm_destroy(lbm_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (void* p : {c->f[0], c->f[1], (void*)c->mask, (void*)c->cls, (void*)c->flags,
                   (void*)c->rec_node, (void*)c->rec_dirs, (void*)c->rec_w,
-                  (void*)c->special, (void*)c->special_rec,
-                  (void*)c->flow_mask, (void*)c->force,
-                  (void*)c->force_partials, (void*)c->red, (void*)c->red_out,
-                  (void*)c->ref_cls, (void*)c->ref_keep, (void*)c->ref_inmask, (void*)c->ref_rxbase,
-                  (void*)c->ref_gsrc, (void*)c->ref_gbeg, (void*)c->ref_gid, (void*)c->ref_gsum,
-                  (void*)c->ref_eidx, (void*)c->ref_ew, (void*)c->ref_es,
-                  (void*)c->ref_partials, c->stage})
+                  (void*)c->flow_mask, (void*)c->force, (void*)c->red, (void*)c->red_out,
+                  c->ref_tables, c->stage})
     if (p) (void)hipFree(p);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -794,19 +567,23 @@ int lbm_upload_points(lbm_ctx* c, const lbm_lattice_point* pts, int64_t count) {
   if ((rc = st.alloc(bytes))) return rc;
   if ((rc = h2d(c, st.p, pts, bytes))) return rc;
   const bool ref = c->cfg.mode == LBM_MODE_REFERENCE;
+  // whether any node's flags change is found on the GPU while they are
+  // written: the geometry tables stay where none does
+  DevBuf changed;
+  int any = 0;
+  if (ref) {
+    if ((rc = changed.alloc(sizeof any))) return rc;
+    LBM_HIP(hipMemsetAsync(changed.p, 0, sizeof any, c->stream));
+  }
   if ((rc = launch_points_in(c->q, device_storage(c->cfg.mode, c->cfg.storage), c->grid,
                              (const lbm_lattice_point*)st.p, c->f[c->cur],
-                             ref ? c->flags : nullptr, c->stream)))
+                             ref ? c->flags : nullptr, (int*)changed.p, c->stream)))
     return rc;
   if ((rc = mirror_buffers(c))) return rc;
-  if (ref) {
-    for (int64_t n = 0; n < count; ++n)
-      c->host_flags[n] =
-          (uint8_t)((pts[n].isInternal ? LBM_FLAG_INTERNAL : 0u) |
-                    (pts[n].isReflected ? LBM_FLAG_REFLECTED : 0u));
-    c->special_dirty = true;
-  }
-  return sync(c);
+  if (!ref) return sync(c);
+  if ((rc = d2h(c, &any, changed.p, sizeof any))) return rc;
+  if (any) c->special_dirty = true;
+  return LBM_OK;
 }
 
 int lbm_download_points(lbm_ctx* c, lbm_lattice_point* pts, int64_t count) {
@@ -909,7 +686,6 @@ int lbm_upload_flags(lbm_ctx* c, const uint8_t* flags) {
   if (int rc = check_ctx(c)) return rc;
   if (int rc = need_mode(c, LBM_MODE_REFERENCE, "lbm_upload_flags")) return rc;
   if (!flags) return fail(LBM_ERR_INVALID, "null flags");
-  std::memcpy(c->host_flags.data(), flags, c->grid.n);
   c->special_dirty = true;
   return h2d(c, c->flags, flags, c->grid.n);
 }
@@ -936,9 +712,6 @@ int lbm_upload_reflections(lbm_ctx* c, int32_t count, const int32_t* node,
   dev_free(c, (void**)&c->rec_dirs, sizeof(uint32_t) * 14 * old);
   dev_free(c, (void**)&c->rec_w, sizeof(float) * 81 * old);
   c->nrec = 0;
-  c->host_rec_node.clear();
-  c->host_rec_dirs.clear();
-  c->host_rec_w.clear();
   c->special_dirty = true;
   const size_t m = (size_t)std::max(count, 1);
   int rc;
@@ -953,9 +726,6 @@ int lbm_upload_reflections(lbm_ctx* c, int32_t count, const int32_t* node,
       return rc;
   }
   c->nrec = count;
-  c->host_rec_node.assign(node, node + count);
-  c->host_rec_dirs.assign(dirs, dirs + 14 * (size_t)count);
-  c->host_rec_w.assign(weights, weights + 81 * (size_t)count);
   // the reflection records usually complete the geometry: build the fused
   // step's receiver tables now rather than in the first step (a later flag
   // change marks them for rebuilding again)

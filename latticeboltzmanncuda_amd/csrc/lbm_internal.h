@@ -188,6 +188,10 @@ int launch_ref_step_full(const Grid& g, const float* A, float* B, float tau,
                          const float* ew, const uint8_t* es, float* partials,
                          float* force, int rev, hipStream_t s);
 int ref_gather_partials(int64_t ngrp);
+// Builds the context's geometry tables (special nodes, receivers) from its
+// flags and reflection records; refuses geometries that the in-place
+// reflection cannot run.
+int build_receivers(lbm_ctx* c);
 int launch_ref_flow(const Grid& g, float* f, const FlowSpec& flow,
                     hipStream_t s);
 int launch_ref_moments(const Grid& g, const float* f, float* rho, float* u,
@@ -196,7 +200,7 @@ int launch_ref_moments(const Grid& g, const float* f, float* rho, float* u,
 // launchers: shared (k_common.hip) --------------------------------------
 int launch_points_in(int q, int storage, const Grid& g,
                      const lbm_lattice_point* pts, void* f, uint8_t* flags,
-                     hipStream_t s);
+                     int* changed, hipStream_t s);
 int launch_points_out(int q, int storage, const Grid& g, const void* f,
                       const uint8_t* flags, lbm_lattice_point* pts,
                       hipStream_t s);
@@ -219,16 +223,15 @@ struct lbm_ctx {
   uint64_t steps_done = 0;   // parity picks the tile order of the next step
   uint64_t params_version = 0;  // bumped when tau or the body force change
   uint8_t* flags = nullptr;  // reference mode
-  std::vector<uint8_t> host_flags;
 
   // reflection records (reference mode)
   int32_t nrec = 0;
   int32_t* rec_node = nullptr;
   uint32_t* rec_dirs = nullptr;
   float* rec_w = nullptr;
-  std::vector<int32_t> host_rec_node;
-  std::vector<uint32_t> host_rec_dirs;  // 14 packed words per record
-  std::vector<float> host_rec_w;        // 81 weights per record
+  // geometry tables of flags and records (build_receivers), one allocation
+  void* ref_tables = nullptr;
+  size_t ref_tables_bytes = 0;
   // nodes with a nonzero flag byte, and their record (or -1)
   int32_t nspecial = 0;
   int32_t* special = nullptr;
@@ -242,7 +245,6 @@ struct lbm_ctx {
   // force register and reduction scratch
   float* force = nullptr;
   float* force_partials = nullptr;
-  int force_partials_cap = 0;
 
   // fused reference step (stream + reflect + collide + flow in one pass):
   // a gather pass sums, for every (receiving node t, direction j), the
@@ -265,7 +267,6 @@ struct lbm_ctx {
   float* ref_ew = nullptr;         // per entry: slot weight W[s]
   uint8_t* ref_es = nullptr;       // per entry: slot s (its force term comes from a table)
   float* ref_partials = nullptr;   // force partials of the gather pass, 3 per wavefront
-  int ref_partials_cap = 0;
   double* red = nullptr;
   int red_cap = 0;
   double* red_out = nullptr;

@@ -157,17 +157,16 @@ int lbm_snapshot_save(lbm_ctx* c, const char* path) {
         (rc = write_all(out.f, buf.data(), h.cls_bytes)))
       return rc;
   } else {
-    if ((rc = write_all(out.f, c->host_flags.data(), N))) return rc;
-    if (h.nrec > 0 &&
-        ((rc = write_all(out.f, c->host_rec_node.data(), 4 * (size_t)h.nrec)) ||
-         (rc = write_all(out.f, c->host_rec_dirs.data(), 4 * 14 * (size_t)h.nrec)) ||
-         (rc = write_all(out.f, c->host_rec_w.data(), 4 * 81 * (size_t)h.nrec))))
+    auto section = [&](const void* src, size_t n) {
+      buf.resize(n);
+      const int e = download(c, buf.data(), src, n);
+      return e ? e : write_all(out.f, buf.data(), n);
+    };
+    const size_t nrec = (size_t)h.nrec;
+    if ((rc = section(c->flags, N)) || (rc = section(c->rec_node, 4 * nrec)) ||
+        (rc = section(c->rec_dirs, 4 * 14 * nrec)) || (rc = section(c->rec_w, 4 * 81 * nrec)) ||
+        (rc = section(c->flow_mask, h.flow_mask_bytes)))
       return rc;
-    if (h.flow_mask_bytes) {
-      buf.resize(N);
-      if ((rc = download(c, buf.data(), c->flow_mask, N)) || (rc = write_all(out.f, buf.data(), N)))
-        return rc;
-    }
   }
   if (std::fclose(out.f) != 0) {
     out.f = nullptr;
