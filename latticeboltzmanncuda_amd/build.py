@@ -47,7 +47,7 @@ HIP_SOURCES = ["lbm_capi.hip", "k_standard.hip", "k_reference.hip",
                "k_common.hip", "lbm_batch.hip", "k_batch.hip",
                "lbm_serve.hip", "k_voxel.hip", "k_receivers.hip",
                "lbm_snapshot.hip",
-               "lbm_exports.hip", "lbm_noalloc.hip"]
+               "lbm_exports.hip", "lbm_noalloc.hip", "lbm_transfer.hip"]
 HOST_SOURCES = ["Constants.cpp", "Geometry.cpp", "Utils.cpp",
                 "FlowCriterion.cpp", "Model.cpp", "Lattice.cpp"]
 CXX = os.environ.get("CXX", "g++")

@@ -566,12 +566,9 @@ int lbm_build_reflections(lbm_ctx* c, const float* vertices, int32_t nv,
                      nf, db, ht, out.at<uint32_t>(o_dirs), out.at<float>(o_w));
   LBM_HIP(hipGetLastError());
   LBM_HIP(hipMemcpyAsync(node, dnode, 4 * (size_t)nrec, hipMemcpyDeviceToHost, c->stream));
-  LBM_HIP(hipMemcpyAsync(dirs, out.at<uint32_t>(o_dirs), 56 * (size_t)nrec, hipMemcpyDeviceToHost,
-                         c->stream));
-  LBM_HIP(hipMemcpyAsync(weights, out.at<float>(o_w), 324 * (size_t)nrec, hipMemcpyDeviceToHost,
-                         c->stream));
-  LBM_HIP(hipStreamSynchronize(c->stream));
-  return LBM_OK;
+  const HostPiece d{dirs, 56 * (size_t)nrec}, w{weights, 324 * (size_t)nrec};
+  if ((rc = copy_to_host(out.at<uint32_t>(o_dirs), &d, 1, c->stream))) return rc;
+  return copy_to_host(out.at<float>(o_w), &w, 1, c->stream);
 }
 
 int lbm_voxelize_mesh(lbm_ctx* c, const float* vertices, int32_t nv,
@@ -631,7 +628,8 @@ int lbm_voxelize_mesh(lbm_ctx* c, const float* vertices, int32_t nv,
                        spacing, dv, df, nf, lo, hi, dout);
   }
   LBM_HIP(hipGetLastError());
-  LBM_HIP(hipMemcpyAsync(inside, dout, (size_t)g.n, hipMemcpyDeviceToHost, c->stream));
+  const HostPiece map{inside, g.n};
+  if ((rc = copy_to_host(dout, &map, 1, c->stream))) return rc;
   unsigned long long total = 0;
   if (closes)
     LBM_HIP(hipMemcpyAsync(&total, mem.at<char>(o_n), 8, hipMemcpyDeviceToHost, c->stream));

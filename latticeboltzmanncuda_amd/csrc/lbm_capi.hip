@@ -233,13 +233,12 @@ int mirror_buffers(lbm_ctx* c) {
 }
 
 int h2d(lbm_ctx* c, void* dst, const void* src, size_t bytes) {
-  LBM_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
-  return sync(c);
+  return copy_to_device(dst, src, bytes, c->stream);
 }
 
 int d2h(lbm_ctx* c, void* dst, const void* src, size_t bytes) {
-  LBM_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-  return sync(c);
+  const HostPiece p{dst, bytes};
+  return copy_to_host(src, &p, 1, c->stream);
 }
 
 int validate_config(const lbm_config* cfg) {
@@ -379,7 +378,7 @@ int step_reference_staged(lbm_ctx* c, int n, int with_force) {
 
 int check_config(const lbm_config* cfg) { return validate_config(cfg); }
 
-int read_moments(lbm_ctx* c, void* stage, float* rho, float* u) {
+int read_moments(lbm_ctx* c, void* stage, float* rho, float* u, bool plain) {
   const size_t N = c->grid.n;
   float* dr = rho ? (float*)stage : nullptr;
   float* du = u ? (float*)stage + (rho ? N : 0) : nullptr;
@@ -390,9 +389,10 @@ int read_moments(lbm_ctx* c, void* stage, float* rho, float* u) {
     rc = launch_std_moments(c->q, device_storage(c->cfg.mode, c->cfg.storage), c->grid,
                             c->f[c->cur], c->mask, c->cfg.force, dr, du, c->stream);
   if (rc) return rc;
-  if (rho && (rc = d2h(c, rho, dr, sizeof(float) * N))) return rc;
-  if (u && (rc = d2h(c, u, du, sizeof(float) * 3 * N))) return rc;
-  return sync(c);
+  // rho and u lie side by side
+  const HostPiece out[2] = {{rho, rho ? sizeof(float) * N : 0}, {u, u ? sizeof(float) * 3 * N : 0}};
+  return plain ? copy_to_host_plain(stage, out, 2, c->stream)
+               : copy_to_host(stage, out, 2, c->stream);
 }
 
 }  // namespace lbm
@@ -493,6 +493,8 @@ int lbm_create(const lbm_config* cfg, void* stream, lbm_ctx** out) {
       return bail(hip_fail(e, "hipMemsetAsync(flags)"));
   }
   if ((rc = sync(c))) return bail(rc);
+  transfer_context(1);
+  c->counted = true;
   *out = c;
   return LBM_OK;
 }
@@ -508,6 +510,7 @@ int lbm_destroy(lbm_ctx* c) {
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
+  if (c->counted) transfer_context(-1);
   delete c;
   return LBM_OK;
 }

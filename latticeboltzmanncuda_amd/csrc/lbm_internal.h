@@ -113,7 +113,20 @@ double cell_reynolds(const lbm_config& cfg);
 // The moments of lbm_moments (rho and / or u, either may be null) staged
 // through the device buffer `stage` -- 4 N bytes for rho, then 12 N for u
 // (12 N from the start when rho is null) -- and copied to the host.
-int read_moments(lbm_ctx* c, void* stage, float* rho, float* u);
+// plain: without the pinned slots of copy_to_host, which it may allocate.
+int read_moments(lbm_ctx* c, void* stage, float* rho, float* u, bool plain = false);
+
+// Copies between device memory and pieces of ordinary host memory laid end
+// to end, in stream order and complete on return (lbm_transfer.hip).
+struct HostPiece {
+  void* p;
+  size_t bytes;
+};
+int copy_to_host(const void* dev, const HostPiece* pieces, int count, hipStream_t s);
+int copy_to_device(void* dev, const void* host, size_t bytes, hipStream_t s);
+int copy_to_host_plain(const void* dev, const HostPiece* pieces, int count, hipStream_t s);
+// a context was made (+1) or goes (-1)
+void transfer_context(int delta);
 
 // error helpers --------------------------------------------------------
 void set_error(const std::string& msg);
@@ -277,6 +290,7 @@ struct lbm_ctx {
 
   hipStream_t stream = nullptr;
   bool own_stream = false;
+  bool counted = false;  // transfer_context(1) was called for it
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int device = 0;
   int64_t device_bytes = 0;

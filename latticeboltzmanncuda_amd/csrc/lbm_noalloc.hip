@@ -73,7 +73,7 @@ int lbm_moments_noalloc(lbm_ctx* c, float* rho, float* u) {
   if (int rc = scratch_address(c->device, &base)) return rc;
   // launches the moments kernels into the array, copies to the host and
   // synchronises the context's stream before the lock is released
-  return read_moments(c, base, rho, u);
+  return read_moments(c, base, rho, u, true);
 }
 
 }  // namespace api

@@ -1,0 +1,322 @@
+// Copies between a caller's ordinary (pageable) host memory and the GPU.
+//
+// The runtime's own copy of pageable memory moves it through one thread and
+// waits for each call.  Here chunks pass through a ring of pinned slots: the
+// GPU fills (or drains) one slot while CPU threads copy others.  The threads
+// of a large copy to the host first touch the pages of the result, which the
+// caller's steps still queued on the GPU mostly hide: a fresh array's page
+// faults cost as much as the copy.  Moments of 256^3 nodes, 268 MB: 26 ms ->
+// 13 ms into a fresh array with nothing queued, 8 ms behind queued steps or
+// into touched pages; of 256 x 128 x 128, 67 MB: 5.7 -> 2.5 ms; of 64^2: 62
+// -> 27 us (one copy for both arrays).
+//
+// Rings (32 MiB each) are taken from a pool that keeps at most kKept of
+// them; each call has a ring to itself, so calls of several threads and
+// streams do not meet.  The pool is emptied when the last context goes.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "lbm_internal.h"
+
+namespace lbm {
+namespace {
+
+constexpr int kSlots = 8;
+// an eighth of the copy, within these: small ones still overlap their two
+// halves, large ones spend little on the chunks' events (268 MB in chunks of
+// 1 MiB: 10.5 ms, of 4 MiB: 8.9)
+constexpr size_t kMinChunk = 512u << 10, kMaxChunk = 4u << 20;
+inline size_t chunk_bytes(size_t bytes) {
+  return std::min(std::max((bytes / kSlots + 4095) / 4096 * 4096, kMinChunk), kMaxChunk);
+}
+constexpr size_t kKept = 2;
+// below this the runtime's copy is as fast (64 KiB: 12 us either way)
+constexpr size_t kDirect = 64u << 10;
+// from here on several threads pay for their start (about 0.1 ms)
+constexpr size_t kThreaded = 8u << 20;
+constexpr int kWorkers = 6;
+// the runtime's upload of pageable memory is as fast up to here (9.4 MB: 355
+// against 485 us, 36 MB: 1350 / 1150, 318 MB: 19.4 / 12 ms)
+constexpr size_t kFeed = 32u << 20;
+
+struct Slots {
+  int device;
+  char* base;
+  hipEvent_t ev[kSlots];
+};
+std::mutex g_pool_mutex;
+std::vector<Slots> g_pool;
+int64_t g_contexts = 0;
+
+void free_slots(const Slots& r) {
+  for (hipEvent_t e : r.ev)
+    if (e) (void)hipEventDestroy(e);
+  if (r.base) (void)hipHostFree(r.base);
+}
+
+// A ring of slots (with an event each) for one call.
+struct Ring {
+  Slots r{};
+  bool ok = false;
+  Ring() {
+    if (hipGetDevice(&r.device) != hipSuccess) return;
+    {
+      std::lock_guard<std::mutex> lk(g_pool_mutex);
+      for (size_t k = 0; k < g_pool.size(); ++k)
+        if (g_pool[k].device == r.device) {
+          r = g_pool[k];
+          g_pool.erase(g_pool.begin() + (std::ptrdiff_t)k);
+          ok = true;
+          return;
+        }
+    }
+    ok = hipHostMalloc((void**)&r.base, kSlots * kMaxChunk, hipHostMallocDefault) == hipSuccess;
+    if (!ok) r.base = nullptr;
+    for (hipEvent_t& e : r.ev)
+      if (ok) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+  }
+  Ring(const Ring&) = delete;
+  Ring& operator=(const Ring&) = delete;
+  ~Ring() {
+    {
+      std::lock_guard<std::mutex> lk(g_pool_mutex);
+      if (ok && g_contexts > 0 && g_pool.size() < kKept) {
+        g_pool.push_back(r);
+        return;
+      }
+    }
+    free_slots(r);
+  }
+  char* slot(size_t j) const { return r.base + (j % kSlots) * kMaxChunk; }
+  hipEvent_t event(size_t j) const { return r.ev[j % kSlots]; }
+};
+
+// Threads that run fn until the object goes; none where they cannot start.
+struct Crew {
+  std::vector<std::thread> t;
+  std::atomic<bool>& stop;
+  template <class Fn>
+  Crew(std::atomic<bool>& s, int n, Fn fn) : stop(s) {
+    t.reserve((size_t)n);
+    for (int k = 0; k < n; ++k) {
+      try {
+        t.emplace_back(fn);
+      } catch (...) {
+        break;
+      }
+    }
+  }
+  ~Crew() {
+    stop.store(true, std::memory_order_release);
+    for (std::thread& x : t) x.join();
+  }
+};
+
+// Bytes [a, b) of the pieces laid end to end, to or from `chunk`.
+void move_pieces(const HostPiece* pieces, int count, size_t a, size_t b, char* chunk, bool out) {
+  size_t at = 0;
+  for (int k = 0; k < count; ++k) {
+    const size_t lo = std::max(a, at), hi = std::min(b, at + pieces[k].bytes);
+    if (lo < hi) {
+      char* host = (char*)pieces[k].p + (lo - at);
+      if (out)
+        std::memcpy(host, chunk + (lo - a), hi - lo);
+      else
+        std::memcpy(chunk + (lo - a), host, hi - lo);
+    }
+    at += pieces[k].bytes;
+  }
+}
+
+int plain(char* dev, const HostPiece* pieces, int count, bool out, hipStream_t s) {
+  for (int k = 0; k < count; ++k) {
+    if (pieces[k].bytes)
+      LBM_HIP(out ? hipMemcpyAsync(pieces[k].p, dev, pieces[k].bytes, hipMemcpyDeviceToHost, s)
+                  : hipMemcpyAsync(dev, pieces[k].p, pieces[k].bytes, hipMemcpyHostToDevice, s));
+    dev += pieces[k].bytes;
+  }
+  LBM_HIP(hipStreamSynchronize(s));
+  return LBM_OK;
+}
+
+void pause() { std::this_thread::yield(); }
+
+// Touches the pages of the pieces without changing what they hold, block by
+// block by the threads that draw them; returns when all blocks are done (a
+// copy into pages that another thread still touches would lose bytes) or
+// stop is set.
+struct Toucher {
+  static constexpr size_t kBlock = 2u << 20, kPage = 4096;
+  const HostPiece* pieces;
+  int count;
+  size_t blocks = 0;
+  std::atomic<size_t> next{0}, done{0};
+  Toucher(const HostPiece* p, int n) : pieces(p), count(n) {
+    for (int k = 0; k < n; ++k) blocks += (p[k].bytes + kBlock - 1) / kBlock;
+  }
+  void block(size_t j) {
+    for (int k = 0; k < count; ++k) {
+      const size_t here = (pieces[k].bytes + kBlock - 1) / kBlock;
+      if (j >= here) {
+        j -= here;
+        continue;
+      }
+      char* p = (char*)pieces[k].p;
+      const size_t end = std::min(pieces[k].bytes, (j + 1) * kBlock);
+      for (size_t i = j * kBlock; i < end; i += kPage) {
+        volatile char* q = p + i;
+        *q = *q;  // a store, which volatile keeps
+      }
+      return;
+    }
+  }
+  void run(const std::atomic<bool>& stop) {
+    for (size_t j; (j = next.fetch_add(1)) < blocks;) {
+      if (!stop.load(std::memory_order_relaxed)) block(j);
+      done.fetch_add(1, std::memory_order_release);
+    }
+    while (done.load(std::memory_order_acquire) < blocks &&
+           !stop.load(std::memory_order_acquire))
+      pause();
+  }
+};
+
+// GPU -> host: slot after slot is filled in stream order; the crew (or this
+// thread) empties those that are there.
+int drain(const char* dev, const HostPiece* pieces, int count, size_t bytes, const Ring& r,
+          hipStream_t s) {
+  const size_t chunk = chunk_bytes(bytes), n = (bytes + chunk - 1) / chunk;
+  auto end = [&](size_t j) { return std::min(bytes, (j + 1) * chunk); };
+  if (n == 1) {
+    LBM_HIP(hipMemcpyAsync(r.slot(0), dev, bytes, hipMemcpyDeviceToHost, s));
+    LBM_HIP(hipStreamSynchronize(s));
+    move_pieces(pieces, count, 0, bytes, r.slot(0), true);
+    return LBM_OK;
+  }
+  auto issue = [&](size_t j) -> hipError_t {
+    const hipError_t e = hipMemcpyAsync(r.slot(j), dev + j * chunk, end(j) - j * chunk,
+                                        hipMemcpyDeviceToHost, s);
+    return e == hipSuccess ? hipEventRecord(r.event(j), s) : e;
+  };
+  std::vector<std::atomic<int>> state(n);  // 1: in its slot, 2: copied out
+  std::atomic<size_t> next{0};
+  std::atomic<bool> stop{false};
+  Toucher toucher(pieces, count);
+  auto copy = [&](size_t j) {
+    move_pieces(pieces, count, j * chunk, end(j), r.slot(j), true);
+    state[j].store(2, std::memory_order_release);
+  };
+  auto work = [&]() {
+    toucher.run(stop);
+    for (;;) {
+      const size_t j = next.fetch_add(1);
+      if (j >= n) return;
+      while (state[j].load(std::memory_order_acquire) == 0) {
+        if (stop.load(std::memory_order_acquire)) return;
+        pause();
+      }
+      copy(j);
+    }
+  };
+  Crew crew(stop, bytes >= kThreaded ? kWorkers : 0, work);
+  for (size_t j = 0; j < n && j < kSlots; ++j) LBM_HIP(issue(j));
+  for (size_t j = 0; j < n; ++j) {
+    LBM_HIP(hipEventSynchronize(r.event(j)));
+    state[j].store(1, std::memory_order_release);
+    if (crew.t.empty()) copy(j);
+    // the slot takes chunk j + kSlots once its own is out; the crew is
+    // several chunks behind at most, so look at the oldest first
+    if (j + kSlots < n) {
+      while (state[j].load(std::memory_order_acquire) != 2) pause();
+      LBM_HIP(issue(j + kSlots));
+    }
+  }
+  for (size_t j = n > kSlots ? n - kSlots : 0; j < n; ++j)
+    while (state[j].load(std::memory_order_acquire) != 2) pause();
+  return LBM_OK;
+}
+
+// Host -> GPU, the other way round.
+int feed(char* dev, const HostPiece* pieces, int count, size_t bytes, const Ring& r,
+         hipStream_t s) {
+  const size_t chunk = chunk_bytes(bytes), n = (bytes + chunk - 1) / chunk;
+  auto end = [&](size_t j) { return std::min(bytes, (j + 1) * chunk); };
+  std::vector<std::atomic<int>> full(n);
+  std::atomic<size_t> next{0}, free_below{std::min<size_t>(n, kSlots)};
+  std::atomic<bool> stop{false};
+  auto fill = [&](size_t j) {
+    move_pieces(pieces, count, j * chunk, end(j), r.slot(j), false);
+    full[j].store(1, std::memory_order_release);
+  };
+  auto work = [&]() {
+    for (;;) {
+      const size_t j = next.fetch_add(1);
+      if (j >= n) return;
+      while (free_below.load(std::memory_order_acquire) <= j) {
+        if (stop.load(std::memory_order_acquire)) return;
+        pause();
+      }
+      fill(j);
+    }
+  };
+  Crew crew(stop, bytes >= kThreaded ? kWorkers : 0, work);
+  for (size_t j = 0; j < n; ++j) {
+    if (j >= kSlots) {
+      LBM_HIP(hipEventSynchronize(r.event(j)));
+      free_below.store(j + 1, std::memory_order_release);
+    }
+    if (crew.t.empty()) fill(j);
+    while (full[j].load(std::memory_order_acquire) == 0) pause();
+    LBM_HIP(hipMemcpyAsync(dev + j * chunk, r.slot(j), end(j) - j * chunk, hipMemcpyHostToDevice, s));
+    LBM_HIP(hipEventRecord(r.event(j), s));
+  }
+  LBM_HIP(hipStreamSynchronize(s));
+  return LBM_OK;
+}
+
+int transfer(char* dev, const HostPiece* pieces, int count, bool out, hipStream_t s) {
+  size_t bytes = 0;
+  for (int k = 0; k < count; ++k) bytes += pieces[k].bytes;
+  if (bytes < (out ? kDirect : kFeed)) return plain(dev, pieces, count, out, s);
+  Ring ring;
+  if (!ring.ok) return plain(dev, pieces, count, out, s);
+  const int rc = out ? drain(dev, pieces, count, bytes, ring, s)
+                     : feed(dev, pieces, count, bytes, ring, s);
+  // after a failure nothing may still move through the slots
+  if (rc) (void)hipStreamSynchronize(s);
+  return rc;
+}
+
+}  // namespace
+
+int copy_to_host(const void* dev, const HostPiece* pieces, int count, hipStream_t s) {
+  return transfer((char*)const_cast<void*>(dev), pieces, count, true, s);
+}
+
+int copy_to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
+  const HostPiece p{const_cast<void*>(host), bytes};
+  return transfer((char*)dev, &p, 1, false, s);
+}
+
+int copy_to_host_plain(const void* dev, const HostPiece* pieces, int count, hipStream_t s) {
+  return plain((char*)const_cast<void*>(dev), pieces, count, true, s);
+}
+
+void transfer_context(int delta) {
+  std::vector<Slots> drop;
+  {
+    std::lock_guard<std::mutex> lk(g_pool_mutex);
+    g_contexts += delta;
+    if (g_contexts == 0) drop.swap(g_pool);
+  }
+  for (const Slots& r : drop) free_slots(r);
+}
+
+}  // namespace lbm

@@ -1,0 +1,86 @@
+"""Copies between host arrays and the GPU through the pinned slots: what goes
+up comes down unchanged, for sizes around the direct copy's limit, one chunk,
+the ring of slots and the threaded copies, from several threads at once, and
+the moments' two arrays (which share their chunks) equal the direct
+read-back's."""
+import sys
+import threading
+
+import numpy as np
+import pytest
+
+from latticeboltzmanncuda_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+# nodes of a D3Q27 FP32 lattice (108 bytes each): 64 KiB, 512 KiB, 8 chunks of
+# 512 KiB, 8 MiB, 32 MiB, each from both sides
+NODES = [1, 606, 607, 4854, 4855, 38836, 38837, 77672, 77673, 310689, 310690,
+         500009]
+
+
+def say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def round_trip(n, seed):
+    f = np.random.default_rng(seed).random(27 * n, np.float32)
+    with capi.Context(capi.make_config(n, 1, 1, lattice=27,
+                                       mode=capi.MODE_REFERENCE)) as c:
+        c.set_populations(f)
+        assert np.array_equal(c.populations(), f)
+        pts = c.download_points()
+        assert np.array_equal(pts["f"], f.reshape(27, n).T)
+        pts["f"] += 1
+        c.upload_points(pts)
+        again = c.download_points()
+        assert np.array_equal(again["f"], pts["f"])
+
+
+@pytest.mark.parametrize("n", NODES)
+def test_round_trip(n):
+    say(f"case: transfer round trip, {n} nodes")
+    round_trip(n, n)
+
+
+def test_round_trips_of_several_threads():
+    say("case: transfers of 4 threads")
+    errors = []
+
+    def work(k):
+        try:
+            for n in (5000 + k, 90000 + k, 1000 + k, 40000 + k):
+                round_trip(n, k)
+        except BaseException as e:  # noqa: BLE001 (reported below)
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+
+
+@pytest.mark.parametrize("dims", [(3, 1000), (31, 1057), (700, 751),
+                                  (1500, 1301)])
+def test_moments_pieces(dims):
+    say(f"case: moments in pieces {dims}")
+    n = dims[0] * dims[1]
+    with capi.Context(capi.make_config(*dims, 1, lattice=capi.D2Q9, tau=0.8,
+                                       periodic=(1, 1, 0))) as c:
+        rng = np.random.default_rng(1)
+        u = 0.02 * (rng.random((3, n)) - 0.5)
+        u[2] = 0
+        c.init_equilibrium(1.0 + 0.01 * rng.random(n), u)
+        c.step(3)
+        rho, vel = c.moments()
+        r2 = np.zeros(n, np.float32)
+        v2 = np.zeros(3 * n, np.float32)
+        capi.check(c.lib.lbm_moments_noalloc(c.h, r2.ctypes.data,
+                                             v2.ctypes.data), "noalloc")
+        assert np.array_equal(rho, r2) and np.array_equal(vel.ravel(), v2)
+        v3 = np.zeros(3 * n, np.float32)
+        capi.check(c.lib.lbm_moments(c.h, None, v3.ctypes.data), "moments")
+        assert np.array_equal(v2, v3)
