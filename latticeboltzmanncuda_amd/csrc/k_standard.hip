@@ -8,7 +8,9 @@
 //
 // The per-node update is std_node_step (lbm_step_node.h); large D2Q9
 // lattices with 16-bit storage take std_group_step instead, 2 or 4 nodes
-// per thread (k_std_stepv, chosen by group_step_width).  Lattices whose
+// per thread (k_std_stepv, chosen by group_step_width).  Several steps of a
+// D2Q9 lattice go in one launch: box by box in LDS for the small ones
+// (k_std_box), as a sweep for the large ones (k_std_sweep).  Lattices whose
 // two population copies exceed the Infinity Cache use non-temporal stores
 // and walk the tiles in opposite orders on consecutive steps; smaller ones
 // use ordinary stores and a fixed order (both measured fastest on MI355X).
@@ -16,6 +18,7 @@
 
 #include <type_traits>
 
+#include "lbm_box.h"
 #include "lbm_internal.h"
 #include "lbm_lattice.h"
 #include "lbm_layout.h"
@@ -78,6 +81,16 @@ __global__ void __launch_bounds__(kBlock)
   const uint32_t n0 = (blk * kBlock + threadIdx.x) * (uint32_t)NV;
   if (n0 >= g.n) return;  // the rows of active groups are whole
   std_group_step<Q, S, NV, LID, NT>(g, A, B, mask, cls, p, n0);
+}
+
+// K steps of a small D2Q9 lattice (box_unit), one box per workgroup.
+template <class X, int S>
+__global__ void __launch_bounds__(X::kThreads)
+    k_std_box(Grid g, const typename Store<S>::T* __restrict__ A,
+              typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
+              const uint32_t* __restrict__ cls, StdParams p) {
+  __shared__ BoxShared<X, typename Store<S>::T> sh;
+  box_unit<X, S>(g, A, B, mask, cls, p, sh, blockIdx.x);
 }
 
 // K steps of a D2Q9 lattice in one pass (sweep_unit), one unit per wavefront.
@@ -409,9 +422,39 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
   return LBM_OK;
 }
 
+namespace {
+// The environment variable asks for steps one at a time.
+bool single_steps() {
+  const char* env = std::getenv("LBM_GROUP_STEP");
+  return env && (env[0] == '0' || env[0] == '1');
+}
+}  // namespace
+
+int std_box_steps(int q, int storage, const Grid& g) {
+  if (q != 9 || single_steps() ||
+      box_wide_count(g) * kBoxWideNodes > box_max_nodes(storage))
+    return 0;
+  return g.n <= box_small_nodes(storage) ? 8 : 4;
+}
+
+int launch_std_box(int k, int storage, const Grid& g, const void* A, void* B,
+                   const uint32_t* mask, const uint32_t* cls, const StdParams& p, hipStream_t s) {
+  const int drc = dispatch_box(storage, g.n, k, [&](auto x, auto st) {
+    using X = decltype(x);
+    constexpr int S = decltype(st)::value;
+    using T = typename Store<S>::T;
+    const uint32_t side = X::kSide;
+    const dim3 grid(((g.nx + side - 1) / side) * ((g.ny + side - 1) / side));
+    hipLaunchKernelGGL((k_std_box<X, S>), grid, dim3(X::kThreads), 0, s, g, (const T*)A, (T*)B,
+                       mask, cls, p);
+  });
+  if (drc) return drc;
+  LBM_HIP(hipGetLastError());
+  return LBM_OK;
+}
+
 bool std_sweeps(int q, int storage, const Grid& g) {
-  const char* env = std::getenv("LBM_GROUP_STEP");  // asks for steps one at a time
-  if (q != 9 || (env && (env[0] == '0' || env[0] == '1'))) return false;
+  if (q != 9 || single_steps()) return false;
   // 16-bit lattices that fit the Infinity Cache are as fast one step at a
   // time (2900 x 1700: 24.2-30.5 against 24.7-28.9 us), larger ones are not
   return storage_bytes(storage) == 2 ? streaming_stores(2 * population_elems(q, g.n) * 2)

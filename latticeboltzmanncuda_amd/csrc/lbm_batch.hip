@@ -235,7 +235,7 @@ int launch_steps(lbm_batch* b, int n) {
     // launches of one step each, or for the D2Q9 lattices passes of up to
     // four; as many passes, odd or even, as there are steps, so that every
     // member's current buffer is the same one
-    const int passes = k == 0 && b->nunits ? sweep_passes(n, true) : n;
+    const int passes = k == 0 && b->nunits ? sweep_passes(n) : n;
     for (int s = 0, left = n; s < passes; ++s) {
       const int steps = (left + (passes - s) - 1) / (passes - s);
       const int rc =

@@ -296,15 +296,23 @@ int rebuild_special(lbm_ctx* c) {
 int step_standard(lbm_ctx* c, int n) {
   const StdParams p = make_std_params(c->cfg);
   const int storage = device_storage(c->cfg.mode, c->cfg.storage);
-  const bool sweeps = n > 1 && std_sweeps(c->q, storage, c->grid);
+  const int box = n > 1 ? std_box_steps(c->q, storage, c->grid) : 0;
+  const bool sweeps = n > 1 && !box && std_sweeps(c->q, storage, c->grid);
   const SweepPlan plan =
       sweeps ? sweep_plan(c->grid, sweep_chunk_rows(
                                        1, [&](size_t) -> const Grid& { return c->grid; }, storage))
              : SweepPlan{};
-  const int passes = sweeps ? sweep_passes(n, false) : n;
+  // As many passes, odd or even, as there are steps: a caller who captures
+  // the launches finds the state in the same buffer as after single steps.
+  // Boxes of 8 steps come in pairs, the rest is spread like a sweep's.
+  const int eights = box == 8 ? n / 16 * 2 : 0;
+  const int passes = eights + (sweeps || box ? sweep_passes(n - 8 * eights) : n);
   for (int s = 0, left = n; s < passes; ++s) {
-    const int k = (left + (passes - s) - 1) / (passes - s);
-    int rc = k > 1 ? launch_std_sweep(k, storage, c->grid, plan, c->f[c->cur], c->f[c->cur ^ 1],
+    const int k = s < eights ? 8 : (left + (passes - s) - 1) / (passes - s);
+    int rc = k > 1 && box
+                 ? launch_std_box(k, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1], c->mask,
+                                  c->cls, p, c->stream)
+             : k > 1 ? launch_std_sweep(k, storage, c->grid, plan, c->f[c->cur], c->f[c->cur ^ 1],
                                       c->mask, p, c->stream)
                    : launch_std_step(c->q, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1],
                                      c->mask, c->cls, p, (int)(c->steps_done & 1), c->stream);

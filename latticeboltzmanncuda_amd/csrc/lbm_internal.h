@@ -148,6 +148,11 @@ int api_exception() noexcept;
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
                     const uint32_t* mask, const uint32_t* cls,
                     const StdParams& p, int rev, hipStream_t s);
+// The most steps that one launch takes of a small D2Q9 lattice (8 or 4;
+// launch_std_box takes 8 or 2 to 4), 0 for the other lattices.
+int std_box_steps(int q, int storage, const Grid& g);
+int launch_std_box(int k, int storage, const Grid& g, const void* A, void* B,
+                   const uint32_t* mask, const uint32_t* cls, const StdParams& p, hipStream_t s);
 // Whether several steps of a lattice are taken in one pass over memory
 // (launch_std_sweep, k of 2 to 4 steps; large D2Q9 lattices).
 struct SweepPlan;

@@ -120,17 +120,19 @@ uint32_t sweep_chunk_rows(size_t count, GridOf&& grid, int storage) {
   return rows;
 }
 
-// Smallest FP32 / FP64 lattice that a single-lattice sweep is faster for
-// (512^2 FP32 6.48 -> 5.04 us per step, 256^2 3.62 -> 3.87); below, too few
-// wavefronts walk too many rows one after another.
+// Smallest FP32 / FP64 lattice that a single-lattice sweep is used for (the
+// lattices below are stepped in boxes, except those too narrow for them:
+// 512^2 FP32 one step at a time 6.48, in sweeps 4.6-5.0, in boxes 3.0 us per
+// step); a smaller one has too few wavefronts, which walk too many rows one
+// after another.
 constexpr uint32_t kSweepMinNodes = 200000;
 
-// Passes for n steps, as even as they can be: n / passes steps each, the
-// first n % passes one more.  At most 4 steps a pass (a fifth stage's
-// registers leave too few wavefronts).  same_parity: as odd or even as n.
-inline int sweep_passes(int n, bool same_parity) {
+// Passes for n steps, as odd or even as n and as even in length as they can
+// be: n / passes steps each, the first n % passes one more.  At most 4 steps
+// a pass (a fifth stage's registers leave too few wavefronts).
+inline int sweep_passes(int n) {
   const int p = (n + 3) / 4;
-  return same_parity && ((p ^ n) & 1) ? p + 1 : p;
+  return ((p ^ n) & 1) ? p + 1 : p;
 }
 
 // v of the next lane (y + 1) / of the previous one (y - 1); 0 past the ends
