@@ -65,6 +65,9 @@ int launch_batch_step(int storage, int cls, bool nt, int block, int grid,
 constexpr int kSweepWaves = 4;
 int launch_batch_sweep(int storage, int k, int grid, const BatchLattice* lats,
                        const BatchTile* units, const uint32_t* nunits, int parity, hipStream_t s);
+// The launch shape that the autotuner chose before for lattices like these
+// (same storage, mix of types and size), if it did.
+bool tuned_shape(int storage, const std::vector<const lbm_config*>& cfgs, int* block, int* grid);
 int launch_batch_residual(int storage, const BatchLattice* lats,
                           const BatchTile* chunks, uint32_t nchunks,
                           double* partials, hipStream_t s);

@@ -319,20 +319,33 @@ int ensure_graph(lbm_batch* b, int chunk) {
 std::mutex g_tune_mutex;
 std::map<std::tuple<int, int, int>, std::pair<int, int>> g_tune_cache;
 
-std::tuple<int, int, int> tune_key(const lbm_batch* b) {
+std::tuple<int, int, int> tune_key(int storage, const std::vector<const lbm_config*>& cfgs) {
   int mix = 0;
   int64_t nodes = 0;
-  for (const lbm_ctx* c : b->slots)
-    if (c) {
-      mix |= c->q == 9 ? 1 : (c->q == 19 ? 2 : 4);
-      nodes += c->grid.n;
-    }
+  for (const lbm_config* c : cfgs) {
+    mix |= c->lattice == 9 ? 1 : (c->lattice == 19 ? 2 : 4);
+    nodes += (int64_t)c->nx * c->ny * c->nz;
+  }
   int lg = 0;
   while ((1ll << (lg + 1)) <= nodes) ++lg;
-  return {b->storage, mix, lg};
+  return {storage, mix, lg};
 }
 
 }  // namespace
+
+namespace lbm {
+
+bool tuned_shape(int storage, const std::vector<const lbm_config*>& cfgs, int* block, int* grid) {
+  if (cfgs.empty()) return false;
+  std::lock_guard<std::mutex> lk(g_tune_mutex);
+  auto it = g_tune_cache.find(tune_key(storage, cfgs));
+  if (it == g_tune_cache.end()) return false;
+  *block = it->second.first;
+  *grid = it->second.second;
+  return true;
+}
+
+}  // namespace lbm
 
 // Entry points of include/lbm.h (exported by lbm_exports.hip).
 namespace lbm {
@@ -580,17 +593,13 @@ int lbm_batch_autotune(lbm_batch* b, int steps, int use_cache, int* block_out,
   if (steps < 2) return fail(LBM_ERR_INVALID, "autotune needs >= 2 steps");
   TraceRange tr("lbm_batch_autotune");
   steps += steps & 1;  // even: members end where they started
-  const auto key = tune_key(b);
-  if (use_cache) {
-    std::lock_guard<std::mutex> lk(g_tune_mutex);
-    auto it = g_tune_cache.find(key);
-    if (it != g_tune_cache.end()) {
-      b->block = it->second.first;
-      b->grid = it->second.second;
-      if (block_out) *block_out = b->block;
-      if (grid_out) *grid_out = b->grid;
-      return LBM_OK;
-    }
+  std::vector<const lbm_config*> cfgs;
+  for (const lbm_ctx* c : b->slots)
+    if (c) cfgs.push_back(&c->cfg);
+  if (use_cache && tuned_shape(b->storage, cfgs, &b->block, &b->grid)) {
+    if (block_out) *block_out = b->block;
+    if (grid_out) *grid_out = b->grid;
+    return LBM_OK;
   }
   float best = 0.0f;
   int best_block = b->block, best_grid = b->grid;
@@ -625,7 +634,7 @@ int lbm_batch_autotune(lbm_batch* b, int steps, int use_cache, int* block_out,
   advance_members(b, launched);  // an even count: buffers end where they began
   {
     std::lock_guard<std::mutex> lk(g_tune_mutex);
-    g_tune_cache[key] = {best_block, best_grid};
+    g_tune_cache[tune_key(b->storage, cfgs)] = {best_block, best_grid};
   }
   if (block_out) *block_out = best_block;
   if (grid_out) *grid_out = best_grid;

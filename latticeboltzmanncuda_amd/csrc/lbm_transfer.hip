@@ -10,9 +10,14 @@
 // into touched pages; of 256 x 128 x 128, 67 MB: 5.7 -> 2.5 ms; of 64^2: 62
 // -> 27 us (one copy for both arrays).
 //
-// Rings (32 MiB each) are taken from a pool that keeps at most kKept of
-// them; each call has a ring to itself, so calls of several threads and
-// streams do not meet.  The pool is emptied when the last context goes.
+// In between, where one thread would fault the pages of a fresh result in one
+// by one, the runtime's copy stays, which pins them at once (2 MB into a
+// fresh array 0.5 against 1.4 ms).
+//
+// Slots (one of 512 KiB for a small copy, a ring of 32 MiB for a large one)
+// are taken from a pool that keeps at most kKept of each; each call has its
+// slots to itself, so calls of several threads and streams do not meet.  The
+// pool is emptied when the last context goes.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,25 +33,26 @@ namespace lbm {
 namespace {
 
 constexpr int kSlots = 8;
-// an eighth of the copy, within these: small ones still overlap their two
-// halves, large ones spend little on the chunks' events (268 MB in chunks of
-// 1 MiB: 10.5 ms, of 4 MiB: 8.9)
-constexpr size_t kMinChunk = 512u << 10, kMaxChunk = 4u << 20;
-inline size_t chunk_bytes(size_t bytes) {
-  return std::min(std::max((bytes / kSlots + 4095) / 4096 * 4096, kMinChunk), kMaxChunk);
-}
 constexpr size_t kKept = 2;
 // below this the runtime's copy is as fast (64 KiB: 12 us either way)
 constexpr size_t kDirect = 64u << 10;
 // from here on several threads pay for their start (about 0.1 ms)
 constexpr size_t kThreaded = 8u << 20;
 constexpr int kWorkers = 6;
+// a small copy takes one slot, a large one chunks of an eighth of it, up to
+// what a slot holds, so that little goes to the chunks' events (268 MB in
+// chunks of 1 MiB: 10.5 ms, of 4 MiB: 8.9)
+constexpr size_t kSmallSlot = 512u << 10, kLargeSlot = 4u << 20;
+inline size_t chunk_bytes(size_t bytes) {
+  return std::min((bytes / kSlots + 4095) / 4096 * 4096, kLargeSlot);
+}
 // the runtime's upload of pageable memory is as fast up to here (9.4 MB: 355
 // against 485 us, 36 MB: 1350 / 1150, 318 MB: 19.4 / 12 ms)
 constexpr size_t kFeed = 32u << 20;
 
 struct Slots {
   int device;
+  bool large;
   char* base;
   hipEvent_t ev[kSlots];
 };
@@ -64,22 +70,24 @@ void free_slots(const Slots& r) {
 struct Ring {
   Slots r{};
   bool ok = false;
-  Ring() {
+  explicit Ring(bool large) {
+    r.large = large;
     if (hipGetDevice(&r.device) != hipSuccess) return;
     {
       std::lock_guard<std::mutex> lk(g_pool_mutex);
       for (size_t k = 0; k < g_pool.size(); ++k)
-        if (g_pool[k].device == r.device) {
+        if (g_pool[k].device == r.device && g_pool[k].large == large) {
           r = g_pool[k];
           g_pool.erase(g_pool.begin() + (std::ptrdiff_t)k);
           ok = true;
           return;
         }
     }
-    ok = hipHostMalloc((void**)&r.base, kSlots * kMaxChunk, hipHostMallocDefault) == hipSuccess;
+    ok = hipHostMalloc((void**)&r.base, large ? kSlots * kLargeSlot : kSmallSlot,
+                       hipHostMallocDefault) == hipSuccess;
     if (!ok) r.base = nullptr;
     for (hipEvent_t& e : r.ev)
-      if (ok) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+      if (ok && large) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (!ok) (void)hipGetLastError();
   }
   Ring(const Ring&) = delete;
@@ -87,14 +95,16 @@ struct Ring {
   ~Ring() {
     {
       std::lock_guard<std::mutex> lk(g_pool_mutex);
-      if (ok && g_contexts > 0 && g_pool.size() < kKept) {
+      size_t kept = 0;
+      for (const Slots& other : g_pool) kept += other.large == r.large;
+      if (ok && g_contexts > 0 && kept < kKept) {
         g_pool.push_back(r);
         return;
       }
     }
     free_slots(r);
   }
-  char* slot(size_t j) const { return r.base + (j % kSlots) * kMaxChunk; }
+  char* slot(size_t j) const { return r.base + (j % kSlots) * kLargeSlot; }
   hipEvent_t event(size_t j) const { return r.ev[j % kSlots]; }
 };
 
@@ -192,14 +202,14 @@ struct Toucher {
 // thread) empties those that are there.
 int drain(const char* dev, const HostPiece* pieces, int count, size_t bytes, const Ring& r,
           hipStream_t s) {
-  const size_t chunk = chunk_bytes(bytes), n = (bytes + chunk - 1) / chunk;
-  auto end = [&](size_t j) { return std::min(bytes, (j + 1) * chunk); };
-  if (n == 1) {
+  if (!r.r.large) {
     LBM_HIP(hipMemcpyAsync(r.slot(0), dev, bytes, hipMemcpyDeviceToHost, s));
     LBM_HIP(hipStreamSynchronize(s));
     move_pieces(pieces, count, 0, bytes, r.slot(0), true);
     return LBM_OK;
   }
+  const size_t chunk = chunk_bytes(bytes), n = (bytes + chunk - 1) / chunk;
+  auto end = [&](size_t j) { return std::min(bytes, (j + 1) * chunk); };
   auto issue = [&](size_t j) -> hipError_t {
     const hipError_t e = hipMemcpyAsync(r.slot(j), dev + j * chunk, end(j) - j * chunk,
                                         hipMemcpyDeviceToHost, s);
@@ -225,7 +235,7 @@ int drain(const char* dev, const HostPiece* pieces, int count, size_t bytes, con
       copy(j);
     }
   };
-  Crew crew(stop, bytes >= kThreaded ? kWorkers : 0, work);
+  Crew crew(stop, kWorkers, work);
   for (size_t j = 0; j < n && j < kSlots; ++j) LBM_HIP(issue(j));
   for (size_t j = 0; j < n; ++j) {
     LBM_HIP(hipEventSynchronize(r.event(j)));
@@ -266,7 +276,7 @@ int feed(char* dev, const HostPiece* pieces, int count, size_t bytes, const Ring
       fill(j);
     }
   };
-  Crew crew(stop, bytes >= kThreaded ? kWorkers : 0, work);
+  Crew crew(stop, kWorkers, work);
   for (size_t j = 0; j < n; ++j) {
     if (j >= kSlots) {
       LBM_HIP(hipEventSynchronize(r.event(j)));
@@ -284,8 +294,10 @@ int feed(char* dev, const HostPiece* pieces, int count, size_t bytes, const Ring
 int transfer(char* dev, const HostPiece* pieces, int count, bool out, hipStream_t s) {
   size_t bytes = 0;
   for (int k = 0; k < count; ++k) bytes += pieces[k].bytes;
-  if (bytes < (out ? kDirect : kFeed)) return plain(dev, pieces, count, out, s);
-  Ring ring;
+  const bool large = bytes >= (out ? kThreaded : kFeed);
+  const bool small = out && bytes >= kDirect && bytes <= kSmallSlot;
+  if (!large && !small) return plain(dev, pieces, count, out, s);
+  Ring ring(large);
   if (!ring.ok) return plain(dev, pieces, count, out, s);
   const int rc = out ? drain(dev, pieces, count, bytes, ring, s)
                      : feed(dev, pieces, count, bytes, ring, s);
