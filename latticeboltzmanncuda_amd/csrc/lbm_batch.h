@@ -80,6 +80,9 @@ struct lbm_batch {
   hipStream_t stream = nullptr;
   bool own_stream = false;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // streams of the classes after the first, made when first needed
+  hipStream_t side[lbm::kBatchClasses] = {};
+  hipEvent_t fork = nullptr, join[lbm::kBatchClasses] = {};
   int device_cus = 0;
 
   double max_cell_re = 0.0;        // admission stability limit, 0 = none
@@ -117,10 +120,10 @@ struct lbm_batch {
   int tables_block = 0;  // block size the tile table was built for
   bool nt = false;       // non-temporal stores: members exceed the Infinity Cache
 
-  // captured chunk
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t graph_exec = nullptr;
-  int graph_chunk = 0, graph_block = 0;
+  // captured chunk, by class
+  hipGraph_t graph[lbm::kBatchClasses] = {};
+  hipGraphExec_t graph_exec[lbm::kBatchClasses] = {};
+  int graph_chunk = 0, graph_block = 0;  // 0 steps: none captured
   bool graph_nt = false;
   const void* graph_lats = nullptr;    // descriptor table the graph reads
   const void* graph_ntiles = nullptr;  // tile counts the graph reads

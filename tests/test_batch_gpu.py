@@ -166,3 +166,30 @@ def test_batch_member_parameter_change_between_chunks():
         c.step(20)
         ref = c.populations()
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("calls", [[(9, 0)], [(10, 0), (35, 0)],
+                                   [(45, 10), (100, 100), (12, 6), (7, 2)]])
+def test_classes_side_by_side_equal_alone(calls):
+    # D2Q9, D3Q19 and D3Q27 members step on streams of their own; a member
+    # read between two calls is complete, and one that leaves and one that
+    # joins find no step under way
+    say(f"case: three lattice types side by side, calls {calls}")
+    specs = mixed_specs()
+    specs.append((capi.make_config(30, 17, 22, lattice=27, tau=0.7,
+                                   periodic=(1, 1, 0)), None))
+    with capi.Batch(capi.STORE_F32) as b:
+        members = [b.add(cfg, solid) for cfg, solid in specs]
+        done = 0
+        for n, chunk in calls:
+            b.step(n, chunk)
+            done += n
+            for k in (0, 4, 6):
+                assert np.array_equal(members[k].populations(),
+                                      run_alone(*specs[k], done))
+        b.remove(members[1])
+        late = b.add(*specs[5])
+        b.step(40, 20)
+        assert np.array_equal(late.populations(), run_alone(*specs[5], 40))
+        assert np.array_equal(members[6].populations(),
+                              run_alone(*specs[6], done + 40))
