@@ -57,12 +57,27 @@ __device__ __forceinline__ uint32_t xcd_run_block(uint32_t w) {
   return (j / kXcdRun) * (8u * kXcdRun) + (w % 8u) * kXcdRun + j % kXcdRun;
 }
 
+// The kernels get the constants of their own storage type only: all three
+// sets are 1.9 KB of arguments, which the host writes for every launch (4.3
+// us a launch with them, 2.6 with one: more than a small lattice's step).
+template <int S>
+using Coef = StepCoef<typename Store<S>::C>;
+template <int S>
+const Coef<S>& coef_of(const StdParams& p) {
+  if constexpr (S == LBM_STORE_F64)
+    return p.cd;
+  else if constexpr (S == LBM_STORE_F16)
+    return p.ch;
+  else
+    return p.cf;
+}
+
 template <int Q, int S, bool LID, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_std_step(Grid g, const typename Store<S>::T* __restrict__ A,
                typename Store<S>::T* __restrict__ B,
                const uint32_t* __restrict__ mask,
-               const uint32_t* __restrict__ cls, StdParams p, int rev) {
+               const uint32_t* __restrict__ cls, Coef<S> p, int rev) {
   const uint32_t w = kXcdRuns<Q, S> ? xcd_run_block(blockIdx.x) : blockIdx.x;
   const uint32_t blk = rev ? gridDim.x - 1 - w : w;
   const uint32_t n = blk * kBlock + threadIdx.x;
@@ -70,12 +85,42 @@ __global__ void __launch_bounds__(kBlock)
   std_node_step<Q, S, LID, NT>(g, A, B, mask, cls, p, n);
 }
 
+// Small 3-D lattices (std_gather_early), one wavefront per workgroup: they
+// have fewer of them than would fill the GPU.  Up to kEarlyNodes, where
+// twice the loads cost less than the latencies: per step, loads in turn
+// against early, D3Q19 24^3 FP32 3.8 -> 3.6 us, 32^3 FP32 3.9 -> 3.5, FP64
+// 5.0 -> 4.2, D3Q27 32^3 FP32 5.0 -> 4.2, FP64 6.3 -> 5.3; 40^3 D3Q19 FP32
+// 4.8 / 5.6.
+constexpr uint32_t kEarlyNodes = 36000;
+template <int Q, int S>
+__global__ void __launch_bounds__(64)
+    k_std_early(Grid g, const typename Store<S>::T* __restrict__ A,
+                typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
+                Coef<S> p) {
+  const uint32_t n = blockIdx.x * 64 + threadIdx.x;
+  if (n >= g.n) return;
+  NodeLoad<Q, S> ld;
+  std_gather_early<Q, S>(g, A, mask, n, ld);
+  using T = typename Store<S>::T;
+  using St = Store<S>;
+  typename St::C gv[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i) gv[i] = St::cvt_u(ld.raw[i]);
+  T* const out = elem(B, ld.own);
+  std_collide_node<Q, S, true>(p, gv, ld.m, ld.solid, [&](auto forced, int i, auto o) {
+    if constexpr (decltype(forced)::value)
+      gstore(out + i * kTile, St::round_sr_u(o, sr_key(St::kShifted ? sr_node_hash(ld.own) : 0u, i)));
+    else
+      gstore(out + i * kTile, round_out<S>(o));
+  });
+}
+
 // Groups of NV nodes per thread (std_group_step).
 template <int Q, int S, int NV, bool LID, bool NT>
 __global__ void __launch_bounds__(kBlock)
     k_std_stepv(Grid g, const typename Store<S>::T* __restrict__ A,
                 typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-                const uint32_t* __restrict__ cls, StdParams p, int rev) {
+                const uint32_t* __restrict__ cls, Coef<S> p, int rev) {
   const uint32_t w = xcd_run_block(blockIdx.x);  // D2Q9 16-bit only
   const uint32_t blk = rev ? gridDim.x - 1 - w : w;
   const uint32_t n0 = (blk * kBlock + threadIdx.x) * (uint32_t)NV;
@@ -88,7 +133,7 @@ template <class X, int S>
 __global__ void __launch_bounds__(X::kThreads)
     k_std_box(Grid g, const typename Store<S>::T* __restrict__ A,
               typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-              const uint32_t* __restrict__ cls, StdParams p) {
+              const uint32_t* __restrict__ cls, Coef<S> p) {
   __shared__ BoxShared<X, typename Store<S>::T> sh;
   box_unit<X, S>(g, A, B, mask, cls, p, sh, blockIdx.x);
 }
@@ -98,7 +143,7 @@ template <int S, int K>
 __global__ void __launch_bounds__(kBlock)
     k_std_sweep(Grid g, SweepPlan pl, const typename Store<S>::T* __restrict__ A,
                 typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-                StdParams p) {
+                Coef<S> p) {
   const uint32_t u =
       __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6));
   if (u >= pl.units) return;
@@ -378,16 +423,16 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
       T* b = (T*)B;
       if (lid && nt)
         hipLaunchKernelGGL((k_std_stepv<9, Tag::S, V, true, true>), gridv, block, 0, s, g, a, b,
-                           mask, cls, p, r);
+                           mask, cls, coef_of<Tag::S>(p), r);
       else if (lid)
         hipLaunchKernelGGL((k_std_stepv<9, Tag::S, V, true, false>), gridv, block, 0, s, g, a, b,
-                           mask, cls, p, r);
+                           mask, cls, coef_of<Tag::S>(p), r);
       else if (nt)
         hipLaunchKernelGGL((k_std_stepv<9, Tag::S, V, false, true>), gridv, block, 0, s, g, a, b,
-                           mask, cls, p, r);
+                           mask, cls, coef_of<Tag::S>(p), r);
       else
         hipLaunchKernelGGL((k_std_stepv<9, Tag::S, V, false, false>), gridv, block, 0, s, g, a,
-                           b, mask, cls, p, r);
+                           b, mask, cls, coef_of<Tag::S>(p), r);
     };
     using Two = std::integral_constant<int, 2>;
     using Four = std::integral_constant<int, 4>;
@@ -395,6 +440,18 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
       width == 4 ? go(QS<9, LBM_STORE_F16>{}, Four{}) : go(QS<9, LBM_STORE_F16>{}, Two{});
     else
       width == 4 ? go(QS<9, LBM_STORE_BF16>{}, Four{}) : go(QS<9, LBM_STORE_BF16>{}, Two{});
+    LBM_HIP(hipGetLastError());
+    return LBM_OK;
+  }
+  if (q != 9 && g.n <= kEarlyNodes) {
+    const int drc = dispatch_qs(q, storage, [&](auto tag) {
+      using Tag = decltype(tag);
+      using T = typename Store<Tag::S>::T;
+      if constexpr (Tag::Q != 9)
+        hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S>), dim3((g.n + 63) / 64), dim3(64), 0, s, g,
+                           (const T*)A, (T*)B, mask, coef_of<Tag::S>(p));
+    });
+    if (drc) return drc;
     LBM_HIP(hipGetLastError());
     return LBM_OK;
   }
@@ -406,16 +463,16 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
     const dim3 grid(kXcdRuns<Tag::Q, Tag::S> ? xcd_run_grid(nb) : nb);
     if (lid && nt)
       hipLaunchKernelGGL((k_std_step<Tag::Q, Tag::S, true, true>), grid, block, 0, s, g, a, b,
-                         mask, cls, p, r);
+                         mask, cls, coef_of<Tag::S>(p), r);
     else if (lid)
       hipLaunchKernelGGL((k_std_step<Tag::Q, Tag::S, true, false>), grid, block, 0, s, g, a, b,
-                         mask, cls, p, r);
+                         mask, cls, coef_of<Tag::S>(p), r);
     else if (nt)
       hipLaunchKernelGGL((k_std_step<Tag::Q, Tag::S, false, true>), grid, block, 0, s, g, a, b,
-                         mask, cls, p, r);
+                         mask, cls, coef_of<Tag::S>(p), r);
     else
       hipLaunchKernelGGL((k_std_step<Tag::Q, Tag::S, false, false>), grid, block, 0, s, g, a, b,
-                         mask, cls, p, r);
+                         mask, cls, coef_of<Tag::S>(p), r);
   });
   if (drc) return drc;
   LBM_HIP(hipGetLastError());
@@ -446,7 +503,7 @@ int launch_std_box(int k, int storage, const Grid& g, const void* A, void* B,
     const uint32_t side = X::kSide;
     const dim3 grid(((g.nx + side - 1) / side) * ((g.ny + side - 1) / side));
     hipLaunchKernelGGL((k_std_box<X, S>), grid, dim3(X::kThreads), 0, s, g, (const T*)A, (T*)B,
-                       mask, cls, p);
+                       mask, cls, coef_of<S>(p));
   });
   if (drc) return drc;
   LBM_HIP(hipGetLastError());
@@ -468,7 +525,7 @@ int launch_std_sweep(int k, int storage, const Grid& g, const SweepPlan& pl, con
     constexpr int S = decltype(tag)::S, K = decltype(steps)::value;
     using T = typename Store<S>::T;
     hipLaunchKernelGGL((k_std_sweep<S, K>), grid, dim3(kBlock), 0, s, g, pl, (const T*)A, (T*)B,
-                       mask, p);
+                       mask, coef_of<S>(p));
   });
   if (drc) return drc;
   LBM_HIP(hipGetLastError());

@@ -84,11 +84,11 @@ constexpr uint32_t kBoxOutside = 1u << 29;
 constexpr uint32_t kBoxSolid = 1u << 28;
 
 // Step s (1..K) of the box whose first row and column are x0 and y0.
-template <class X, int S, int s>
+template <class X, int S, int s, class P>
 __device__ __forceinline__ void box_steps(const Grid& g, const typename Store<S>::T* __restrict__ A,
                                           typename Store<S>::T* __restrict__ B,
                                           const uint32_t* __restrict__ mask,
-                                          const uint32_t* __restrict__ cls, const StdParams& p,
+                                          const uint32_t* __restrict__ cls, const P& p,
                                           BoxShared<X, typename Store<S>::T>& sh, uint32_t x0,
                                           uint32_t y0) {
   using L = Lat<9>;
@@ -157,11 +157,11 @@ __device__ __forceinline__ void box_steps(const Grid& g, const typename Store<S>
 
 // K steps of box u of a lattice (boxes lie along y first), read from A,
 // written to B.
-template <class X, int S>
+template <class X, int S, class P>
 __device__ __forceinline__ void box_unit(const Grid& g, const typename Store<S>::T* __restrict__ A,
                                          typename Store<S>::T* __restrict__ B,
                                          const uint32_t* __restrict__ mask,
-                                         const uint32_t* __restrict__ cls, const StdParams& p,
+                                         const uint32_t* __restrict__ cls, const P& p,
                                          BoxShared<X, typename Store<S>::T>& sh, uint32_t u) {
   const uint32_t across = (g.ny + X::kSide - 1) / X::kSide;
   const uint32_t bx = u / across;

@@ -72,6 +72,13 @@ __device__ __forceinline__ const StepCoef<typename Store<S>::C>& step_coef(const
     return p.cf;
 }
 
+// (the single-lattice kernels get them as their argument)
+template <int S>
+__device__ __forceinline__ const StepCoef<typename Store<S>::C>& step_coef(
+    const StepCoef<typename Store<S>::C>& k) {
+  return k;
+}
+
 // 1 / r: IEEE division in FP64; in FP32 the hardware reciprocal refined by
 // one Newton-Raphson step (error below one unit in the last place)
 __device__ __forceinline__ double recip(double r) { return 1.0 / r; }
@@ -291,6 +298,48 @@ __device__ __forceinline__ void std_gather(const Grid& g,
   }
 }
 
+// The same for a small 3-D lattice, whose step is one chain of latencies:
+// the pulled and the node's own populations are loaded while the link mask
+// is on its way, and chosen from when it is there (class, then mask, then
+// populations are three loads one after another).
+template <int Q, int S>
+__device__ __forceinline__ void std_gather_early(const Grid& g,
+                                                 const typename Store<S>::T* __restrict__ A,
+                                                 const uint32_t* __restrict__ mask, uint32_t n,
+                                                 NodeLoad<Q, S>& ld) {
+  using L = Lat<Q>;
+  using T = typename Store<S>::T;
+  const uint32_t mw = gload(mask + n);
+  ld.own = pidx<Q>(n, 0);
+  ld.pop_bytes = 0;
+  T back[Q];
+  const T* const own = elem(A, ld.own);
+#pragma unroll
+  for (int i = 1; i < Q; ++i) back[i] = gload(own + L::INV[i] * kTile);
+  // offsets (mod 2^32) to the source nodes, wrapped along every axis
+  uint32_t x, y, z;
+  decode_node(g, n, x, y, z);
+  const uint32_t plane = g.ny * g.nz;
+  const uint32_t ox[3] = {x + 1 == g.nx ? plane - g.n : plane, 0u,
+                          x == 0 ? g.n - plane : 0u - plane};
+  const uint32_t oy[3] = {y + 1 == g.ny ? g.nz - plane : g.nz, 0u,
+                          y == 0 ? plane - g.nz : 0u - g.nz};
+  const uint32_t oz[3] = {z + 1 == g.nz ? 1u - g.nz : 1u, 0u, z == 0 ? g.nz - 1u : 0u - 1u};
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const uint32_t src = n + ox[L::E[i][0] + 1] + oy[L::E[i][1] + 1] + oz[L::E[i][2] + 1];
+    ld.raw[i] = gload(elem(A, pidx<Q>(src, i)));
+  }
+  // both are to be loaded: a choice between two loads would become one load
+  // of a chosen address, which waits for the mask
+#pragma unroll
+  for (int i = 1; i < Q; ++i) asm("" : "+v"(back[i]), "+v"(ld.raw[i]));
+  ld.solid = (mw & LBM_MASK_SOLID) != 0u;
+  ld.m = mw & ~LBM_MASK_SOLID;
+#pragma unroll
+  for (int i = 1; i < Q; ++i) ld.raw[i] = ((ld.m >> i) & 1u) ? back[i] : ld.raw[i];
+}
+
 // s * b + c rounded once to FP16 (v_fma_mixlo_f16; s is uniform).  Written
 // out because the compiler folds the conversion into the fma in some
 // surroundings and not in others, which rounds twice: every kernel has to
@@ -393,8 +442,8 @@ __device__ __forceinline__ void std_relax(const StepCoef<typename Store<S>::C>& 
 // or read from the lattice's constants (2).  SOLID: whether the wavefront
 // may hold solid nodes whose outputs matter (0: no, 1: yes, 2: found out
 // here).
-template <int Q, int S, bool LID, int FORCE = 2, int SOLID = 2, class Emit>
-__device__ __forceinline__ void std_collide_node(const StdParams& p,
+template <int Q, int S, bool LID, int FORCE = 2, int SOLID = 2, class P, class Emit>
+__device__ __forceinline__ void std_collide_node(const P& p,
                                                  typename Store<S>::C (&gv)[Q], uint32_t m,
                                                  bool solid, Emit&& emit) {
   // a * b + c is fused only where one source expression has that form, so
@@ -476,8 +525,8 @@ __device__ __forceinline__ void std_collide_node(const StdParams& p,
 }
 
 // Phase 2: collide the loaded node and store its Q post-collision values.
-template <int Q, int S, bool LID, bool NT>
-__device__ __forceinline__ void std_collide(const StdParams& p,
+template <int Q, int S, bool LID, bool NT, class P>
+__device__ __forceinline__ void std_collide(const P& p,
                                             typename Store<S>::T* __restrict__ B,
                                             const NodeLoad<Q, S>& ld) {
   using St = Store<S>;
@@ -509,11 +558,11 @@ __device__ __forceinline__ void std_collide(const StdParams& p,
   });
 }
 
-template <int Q, int S, bool LID, bool NT = false>
+template <int Q, int S, bool LID, bool NT = false, class P>
 __device__ __forceinline__ void std_node_step(
     const Grid& g, const typename Store<S>::T* __restrict__ A,
     typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-    const uint32_t* __restrict__ cls, const StdParams& p, uint32_t n) {
+    const uint32_t* __restrict__ cls, const P& p, uint32_t n) {
   NodeLoad<Q, S> ld;
   std_gather<Q, S>(g, A, mask, cls, n, ld);
   std_collide<Q, S, LID, NT>(p, B, ld);
@@ -584,11 +633,11 @@ __device__ __forceinline__ T lane_value(T v, int lane) {
   }
 }
 
-template <int Q, int S, int NV, bool LID, bool NT>
+template <int Q, int S, int NV, bool LID, bool NT, class P>
 __device__ __forceinline__ void std_group_step(
     const Grid& g, const typename Store<S>::T* __restrict__ A,
     typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-    const uint32_t* __restrict__ cls, const StdParams& p, uint32_t n0) {
+    const uint32_t* __restrict__ cls, const P& p, uint32_t n0) {
   using L = Lat<Q>;
   using St = Store<S>;
   using T = typename St::T;

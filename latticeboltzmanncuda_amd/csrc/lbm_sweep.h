@@ -225,12 +225,12 @@ __device__ __forceinline__ void sweep_load(const Grid& g,
 }
 
 // The unit `u` of a lattice: K steps of its rows, read from A, written to B.
-template <int S, int K, int FORCE>
+template <int S, int K, int FORCE, class Par>
 __device__ __forceinline__ void sweep_rows(const Grid& g, const SweepPlan& pl,
                                            const typename Store<S>::T* __restrict__ A,
                                            typename Store<S>::T* __restrict__ B,
                                            const uint32_t* __restrict__ mask,
-                                           const StdParams& p, uint32_t u) {
+                                           const Par& p, uint32_t u) {
 #pragma clang fp contract(on)
   using St = Store<S>;
   using T = typename St::T;
@@ -401,12 +401,12 @@ __device__ __forceinline__ void sweep_rows(const Grid& g, const SweepPlan& pl,
   }
 }
 
-template <int S, int K>
+template <int S, int K, class Par>
 __device__ __forceinline__ void sweep_unit(const Grid& g, const SweepPlan& pl,
                                            const typename Store<S>::T* __restrict__ A,
                                            typename Store<S>::T* __restrict__ B,
                                            const uint32_t* __restrict__ mask,
-                                           const StdParams& p, uint32_t u) {
+                                           const Par& p, uint32_t u) {
   if (step_coef<S>(p).forced)
     sweep_rows<S, K, 1>(g, pl, A, B, mask, p, u);
   else

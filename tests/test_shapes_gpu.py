@@ -148,3 +148,42 @@ def test_step_matches_batch_and_oracle(q, dims, per, pat, lid, force,
     # result one 16-bit step apart where the FP32 collisions round
     # differently
     assert err < (1e-6 if storage == F32 else 2e-3)
+
+
+# small 3-D lattices read pulled and own populations ahead of their link
+# masks (up to 36000 nodes); a batch of them does not
+EARLY_DIMS = [(1, 1, 1), (2, 1, 65), (64, 3, 1), (7, 9, 11), (33, 33, 33),
+              (36, 20, 50), (30, 30, 41)]
+
+
+@pytest.mark.parametrize("q", [19, 27])
+@pytest.mark.parametrize("storage", [capi.STORE_F32, capi.STORE_F64,
+                                     capi.STORE_F16, capi.STORE_BF16])
+def test_small_3d_equals_batch(q, storage):
+    for k, dims in enumerate(EARLY_DIMS):
+        print(f"case: D3Q{q} {dims} storage {storage}", flush=True)
+        rng = np.random.default_rng(k)
+        n = dims[0] * dims[1] * dims[2]
+        per = ((1, 0, 0), (0, 1, 0), (1, 0, 1), (1, 1, 1), (0, 0, 0),
+               (0, 0, 1), (1, 0, 0))[k]
+        kw = dict(lid_face=3, lid_u=(0.05, 0, 0.01)) if not per[1] else {}
+        cfg = capi.make_config(*dims, lattice=q, storage=storage, tau=0.7,
+                               periodic=per, force=(1e-5 * (k % 2), 0, 2e-6),
+                               **kw)
+        solid = (rng.random(n) < 0.15).astype(np.uint8) if k % 3 else None
+        rho = 1.0 + 0.01 * rng.random(n)
+        u = 0.02 * (rng.random((3, n)) - 0.5)
+        got = []
+        with capi.Batch(storage) as b:
+            m = b.add(cfg, solid)
+            m.init_equilibrium(rho, u)
+            b.step(11)
+            got.append(m.populations(np.float64))
+        with capi.Context(cfg) as c:
+            if solid is not None:
+                c.upload_solid(solid)
+            c.init_equilibrium(rho, u)
+            c.step(11)
+            got.append(c.populations(np.float64))
+        assert np.isfinite(got[0]).all()
+        assert np.array_equal(*got)
