@@ -92,11 +92,32 @@ __global__ void __launch_bounds__(kBlock)
 // 5.0 -> 4.2, D3Q27 32^3 FP32 5.0 -> 4.2, FP64 6.3 -> 5.3; 40^3 D3Q19 FP32
 // 4.8 / 5.6.
 constexpr uint32_t kEarlyNodes = 36000;
-template <int Q, int S>
+
+// The step constants as a kernel's argument, or where k_put_coef left them:
+// many steps of a small lattice are bound by the host, which writes every
+// launch's arguments (32^3 FP32, 1000 steps: 4.1 us a launch with 0.5 KB of
+// them, 2.5 with a pointer; the step on the GPU 3.5).
+template <int S>
+struct CoefValue {
+  Coef<S> k;
+  __device__ const Coef<S>& get() const { return k; }
+};
+template <int S>
+struct CoefPointer {
+  const Coef<S>* k;
+  __device__ const Coef<S>& get() const { return *k; }
+};
+template <int S>
+__global__ void __launch_bounds__(64) k_put_coef(Coef<S> k, Coef<S>* out) {
+  if (threadIdx.x == 0) *out = k;
+}
+
+template <int Q, int S, class Args>
 __global__ void __launch_bounds__(64)
     k_std_early(Grid g, const typename Store<S>::T* __restrict__ A,
                 typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-                Coef<S> p) {
+                Args args) {
+  const Coef<S>& p = args.get();
   const uint32_t n = blockIdx.x * 64 + threadIdx.x;
   if (n >= g.n) return;
   NodeLoad<Q, S> ld;
@@ -403,9 +424,22 @@ inline unsigned blocks_for(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 
 }  // namespace
 
+bool std_takes_coef(int q, const Grid& g) { return q != 9 && g.n <= kEarlyNodes; }
+
+int launch_put_coef(int q, int storage, const StdParams& p, void* coef, hipStream_t s) {
+  const int drc = dispatch_qs(q, storage, [&](auto tag) {
+    constexpr int S = decltype(tag)::S;
+    static_assert(sizeof(Coef<S>) <= kCoefBytes, "the context keeps room for them");
+    hipLaunchKernelGGL((k_put_coef<S>), dim3(1), dim3(64), 0, s, coef_of<S>(p), (Coef<S>*)coef);
+  });
+  if (drc) return drc;
+  LBM_HIP(hipGetLastError());
+  return LBM_OK;
+}
+
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
                     const uint32_t* mask, const uint32_t* cls,
-                    const StdParams& p, int rev, hipStream_t s) {
+                    const StdParams& p, int rev, hipStream_t s, const void* coef) {
   const unsigned nb = blocks_for(g.n);
   const bool lid = p.lid_axis >= 0;
   const bool nt = streaming_stores(2 * population_elems(q, g.n) * storage_bytes(storage));
@@ -447,9 +481,17 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
     const int drc = dispatch_qs(q, storage, [&](auto tag) {
       using Tag = decltype(tag);
       using T = typename Store<Tag::S>::T;
-      if constexpr (Tag::Q != 9)
-        hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S>), dim3((g.n + 63) / 64), dim3(64), 0, s, g,
-                           (const T*)A, (T*)B, mask, coef_of<Tag::S>(p));
+      const dim3 grid((g.n + 63) / 64);
+      if constexpr (Tag::Q != 9) {
+        using Value = CoefValue<Tag::S>;
+        using Pointer = CoefPointer<Tag::S>;
+        if (coef)
+          hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S, Pointer>), grid, dim3(64), 0, s, g,
+                             (const T*)A, (T*)B, mask, Pointer{(const Coef<Tag::S>*)coef});
+        else
+          hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S, Value>), grid, dim3(64), 0, s, g,
+                             (const T*)A, (T*)B, mask, Value{coef_of<Tag::S>(p)});
+      }
     });
     if (drc) return drc;
     LBM_HIP(hipGetLastError());

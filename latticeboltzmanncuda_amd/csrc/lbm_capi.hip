@@ -293,6 +293,10 @@ int rebuild_special(lbm_ctx* c) {
   return LBM_OK;
 }
 
+// From this many steps on one launch more is worth the smaller ones (about
+// 1 us of host time each against 3 to 4 us).
+constexpr int kPutSteps = 16;
+
 int step_standard(lbm_ctx* c, int n) {
   const StdParams p = make_std_params(c->cfg);
   const int storage = device_storage(c->cfg.mode, c->cfg.storage);
@@ -307,6 +311,14 @@ int step_standard(lbm_ctx* c, int n) {
   // Boxes of 8 steps come in pairs, the rest is spread like a sweep's.
   const int eights = box == 8 ? n / 16 * 2 : 0;
   const int passes = eights + (sweeps || box ? sweep_passes(n - 8 * eights) : n);
+  // the constants as they are now, for this call's launches alone: whoever
+  // changes them, or captures the call, finds what a launch with them as
+  // arguments would do
+  const void* coef = nullptr;
+  if (n >= kPutSteps && std_takes_coef(c->q, c->grid)) {
+    if (int rc = launch_put_coef(c->q, storage, p, c->coef, c->stream)) return rc;
+    coef = c->coef;
+  }
   for (int s = 0, left = n; s < passes; ++s) {
     const int k = s < eights ? 8 : (left + (passes - s) - 1) / (passes - s);
     int rc = k > 1 && box
@@ -315,7 +327,7 @@ int step_standard(lbm_ctx* c, int n) {
              : k > 1 ? launch_std_sweep(k, storage, c->grid, plan, c->f[c->cur], c->f[c->cur ^ 1],
                                       c->mask, p, c->stream)
                    : launch_std_step(c->q, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1],
-                                     c->mask, c->cls, p, (int)(c->steps_done & 1), c->stream);
+                                     c->mask, c->cls, p, (int)(c->steps_done & 1), c->stream, coef);
     if (rc) return rc;
     c->cur ^= 1;
     c->steps_done += k;
@@ -482,8 +494,10 @@ int lbm_create(const lbm_config* cfg, void* stream, lbm_ctx** out) {
   c->red_cap = (int)std::min<uint32_t>(1024u, (g.n + 255) / 256);
   if ((rc = dev_alloc(c, (void**)&c->red, sizeof(double) * 4 * c->red_cap, "hipMalloc(reduction)")))
     return bail(rc);
-  if ((rc = dev_alloc(c, (void**)&c->red_out, sizeof(double) * 4, "hipMalloc(reduction)")))
+  // the sums, and room for the step constants behind them
+  if ((rc = dev_alloc(c, (void**)&c->red_out, 4 * sizeof(double) + kCoefBytes, "hipMalloc(reduction)")))
     return bail(rc);
+  c->coef = (char*)c->red_out + 4 * sizeof(double);
   if (cfg->mode == LBM_MODE_STANDARD) {
     if ((rc = dev_alloc(c, (void**)&c->mask, (has_mask16(*cfg) ? 6 : 4) * (size_t)g.n,
                         "hipMalloc(mask)")))

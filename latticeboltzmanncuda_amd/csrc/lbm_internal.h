@@ -147,7 +147,13 @@ int api_exception() noexcept;
 // launchers: standard mode (k_standard.hip) -----------------------------
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
                     const uint32_t* mask, const uint32_t* cls,
-                    const StdParams& p, int rev, hipStream_t s);
+                    const StdParams& p, int rev, hipStream_t s, const void* coef = nullptr);
+// Lattices whose steps can read their constants from device memory
+// (launch_std_step's coef), once launch_put_coef has written them there in
+// stream order: for calls of many steps, whose launches then carry less.
+constexpr size_t kCoefBytes = 960;
+bool std_takes_coef(int q, const Grid& g);
+int launch_put_coef(int q, int storage, const StdParams& p, void* coef, hipStream_t s);
 // The most steps that one launch takes of a small D2Q9 lattice (8 or 4;
 // launch_std_box takes 8 or 2 to 4), 0 for the other lattices.
 int std_box_steps(int q, int storage, const Grid& g);
@@ -288,6 +294,7 @@ struct lbm_ctx {
   double* red = nullptr;
   int red_cap = 0;
   double* red_out = nullptr;
+  void* coef = nullptr;  // kCoefBytes for launch_put_coef, behind red_out's sums
   // device staging of lbm_moments (rho and u), allocated by its first call
   // and kept, so later calls allocate nothing
   void* stage = nullptr;

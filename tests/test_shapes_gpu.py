@@ -187,3 +187,25 @@ def test_small_3d_equals_batch(q, storage):
             got.append(c.populations(np.float64))
         assert np.isfinite(got[0]).all()
         assert np.array_equal(*got)
+
+
+def test_small_3d_constants_are_those_of_the_call():
+    # calls of many steps read their constants from device memory, calls of
+    # few from their arguments: parameters changed between queued calls
+    print("case: small 3-D lattice, parameters changed between calls",
+          flush=True)
+    cfg = capi.make_config(20, 17, 19, lattice=19, storage=capi.STORE_F32,
+                           tau=0.7, periodic=(1, 1, 1))
+    calls = [(16, 0.6, 1e-4), (15, 0.8, 0.0), (40, 1.1, -2e-4), (1, 0.9, 1e-5),
+             (17, 0.55, 3e-4)]
+    got = []
+    for single in (False, True):
+        with capi.Context(cfg) as c:
+            c.init_equilibrium()
+            for n, tau, fx in calls:
+                c.set_tau(tau)
+                c.set_body_force((fx, 0, 1e-5))
+                for k in ([1] * n if single else [n]):
+                    c.step(k)
+            got.append(c.populations())
+    assert np.array_equal(*got)
