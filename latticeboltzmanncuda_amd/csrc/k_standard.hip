@@ -10,7 +10,8 @@
 // lattices with 16-bit storage take std_group_step instead, 2 or 4 nodes
 // per thread (k_std_stepv, chosen by group_step_width).  Several steps of a
 // D2Q9 lattice go in one launch: box by box in LDS for the small ones
-// (k_std_box), as a sweep for the large ones (k_std_sweep).  Lattices whose
+// (k_std_box), as a sweep for the large ones (k_std_sweep); two steps of a
+// large D3Q19 lattice go in one pass along x (k_std_march).  Lattices whose
 // two population copies exceed the Infinity Cache use non-temporal stores
 // and walk the tiles in opposite orders on consecutive steps; smaller ones
 // use ordinary stores and a fixed order (both measured fastest on MI355X).
@@ -22,6 +23,7 @@
 #include "lbm_internal.h"
 #include "lbm_lattice.h"
 #include "lbm_layout.h"
+#include "lbm_march.h"
 #include "lbm_step_node.h"
 #include "lbm_store.h"
 #include "lbm_sweep.h"
@@ -83,6 +85,21 @@ __global__ void __launch_bounds__(kBlock)
   const uint32_t n = blk * kBlock + threadIdx.x;
   if (n >= g.n) return;
   std_node_step<Q, S, LID, NT>(g, A, B, mask, cls, p, n);
+}
+
+// Two steps of a large D3Q19 lattice in one pass (march_unit).  Workgroup w
+// runs on XCD w % 8: each XCD takes a contiguous eighth of the columns, whose
+// rims are read twice, mostly through its L2 (256 x 128 x 128 FP32 1 %, 121 x
+// 67 x 93 FP64 5 % faster).
+template <int S, bool LID, bool NT>
+__global__ void __launch_bounds__(march_threads(sizeof(typename Store<S>::T)))
+    k_std_march(Grid g, MarchPlan pl, const typename Store<S>::T* __restrict__ A,
+                typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
+                Coef<S> p) {
+  __shared__ MarchShared<typename Store<S>::T> sh;
+  const uint32_t w = blockIdx.x, eighth = gridDim.x / 8;
+  const uint32_t u = w < 8 * eighth ? (w % 8) * eighth + w / 8 : w;
+  march_unit<S, LID, NT>(g, pl, A, B, mask, p, sh, u);
 }
 
 // Small 3-D lattices (std_gather_early), one wavefront per workgroup: they
@@ -423,6 +440,43 @@ inline unsigned blocks_for(uint32_t n) { return (n + kBlock - 1) / kBlock; }
 
 
 }  // namespace
+
+bool std_marches(int q, int storage, const Grid& g, MarchPlan* plan) {
+  if (q != 19 || storage_bytes(storage) == 2 || g.n < kMarchMinNodes) return false;
+  double cost;
+  *plan = march_plan(g, storage_bytes(storage), &cost);
+  return march_pays(g, cost);
+}
+
+int launch_std_march(int storage, const Grid& g, const MarchPlan& pl, const void* A, void* B,
+                     const uint32_t* mask, const StdParams& p, hipStream_t s) {
+  const dim3 grid(pl.strips * pl.bands * pl.chunks);
+  // non-temporal stores where rows are whole tiles (128^3 FP32 41.0 -> 38.4
+  // us); others share cache lines with the next column's (100^3 20.6 -> 24.0)
+  const bool nt = pl.strips == 1 && g.nz % kTile == 0;
+  auto go = [&](auto st, auto lid, auto n) {
+    constexpr int S = decltype(st)::value;
+    using T = typename Store<S>::T;
+    hipLaunchKernelGGL((k_std_march<S, decltype(lid)::value, decltype(n)::value>), grid,
+                       dim3(march_threads(sizeof(T))), 0, s, g, pl, (const T*)A, (T*)B, mask,
+                       coef_of<S>(p));
+  };
+  auto by_form = [&](auto st) {
+    if (p.lid_axis >= 0)
+      nt ? go(st, std::true_type{}, std::true_type{}) : go(st, std::true_type{}, std::false_type{});
+    else
+      nt ? go(st, std::false_type{}, std::true_type{})
+         : go(st, std::false_type{}, std::false_type{});
+  };
+  if (storage == kStoreF32Shifted)
+    by_form(std::integral_constant<int, kStoreF32Shifted>{});
+  else if (storage == LBM_STORE_F64)
+    by_form(std::integral_constant<int, LBM_STORE_F64>{});
+  else
+    return fail(LBM_ERR_UNSUPPORTED, "storage not built");
+  LBM_HIP(hipGetLastError());
+  return LBM_OK;
+}
 
 bool std_takes_coef(int q, const Grid& g) { return q != 9 && g.n <= kEarlyNodes; }
 

@@ -21,6 +21,7 @@
 #include "lbm_lattice.h"
 #include "lbm_layout.h"
 #include "lbm_store.h"
+#include "lbm_march.h"
 #include "lbm_sweep.h"
 
 namespace lbm {
@@ -309,8 +310,11 @@ int step_standard(lbm_ctx* c, int n) {
   // As many passes, odd or even, as there are steps: a caller who captures
   // the launches finds the state in the same buffer as after single steps.
   // Boxes of 8 steps come in pairs, the rest is spread like a sweep's.
+  // So do the marches of two.
+  MarchPlan march{};
+  const int pairs = n >= 4 && std_marches(c->q, storage, c->grid, &march) ? n / 4 * 2 : 0;
   const int eights = box == 8 ? n / 16 * 2 : 0;
-  const int passes = eights + (sweeps || box ? sweep_passes(n - 8 * eights) : n);
+  const int passes = pairs ? n - pairs : eights + (sweeps || box ? sweep_passes(n - 8 * eights) : n);
   // the constants as they are now, for this call's launches alone: whoever
   // changes them, or captures the call, finds what a launch with them as
   // arguments would do
@@ -320,8 +324,11 @@ int step_standard(lbm_ctx* c, int n) {
     coef = c->coef;
   }
   for (int s = 0, left = n; s < passes; ++s) {
-    const int k = s < eights ? 8 : (left + (passes - s) - 1) / (passes - s);
-    int rc = k > 1 && box
+    const int k = s < pairs ? 2 : s < eights ? 8 : (left + (passes - s) - 1) / (passes - s);
+    int rc = s < pairs
+                 ? launch_std_march(storage, c->grid, march, c->f[c->cur], c->f[c->cur ^ 1],
+                                    c->mask, p, c->stream)
+             : k > 1 && box
                  ? launch_std_box(k, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1], c->mask,
                                   c->cls, p, c->stream)
              : k > 1 ? launch_std_sweep(k, storage, c->grid, plan, c->f[c->cur], c->f[c->cur ^ 1],

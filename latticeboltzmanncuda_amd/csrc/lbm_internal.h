@@ -159,6 +159,12 @@ int launch_put_coef(int q, int storage, const StdParams& p, void* coef, hipStrea
 int std_box_steps(int q, int storage, const Grid& g);
 int launch_std_box(int k, int storage, const Grid& g, const void* A, void* B,
                    const uint32_t* mask, const uint32_t* cls, const StdParams& p, hipStream_t s);
+// Whether two steps of a lattice are taken in one pass (large D3Q19 lattices
+// in FP32 or FP64), and how it is cut for that.
+struct MarchPlan;
+bool std_marches(int q, int storage, const Grid& g, MarchPlan* plan);
+int launch_std_march(int storage, const Grid& g, const MarchPlan& pl, const void* A, void* B,
+                     const uint32_t* mask, const StdParams& p, hipStream_t s);
 // Whether several steps of a lattice are taken in one pass over memory
 // (launch_std_sweep, k of 2 to 4 steps; large D2Q9 lattices).
 struct SweepPlan;
