@@ -445,7 +445,7 @@ bool std_marches(int q, int storage, const Grid& g, MarchPlan* plan) {
   if (q != 19 || storage_bytes(storage) == 2 || g.n < kMarchMinNodes) return false;
   double cost;
   *plan = march_plan(g, storage_bytes(storage), &cost);
-  return march_pays(g, cost);
+  return march_pays(g, storage_bytes(storage), cost);
 }
 
 int launch_std_march(int storage, const Grid& g, const MarchPlan& pl, const void* A, void* B,

@@ -17,8 +17,9 @@
 // What it costs: the outermost rows (and, where a row does not fit, the ends
 // in z) are computed by two workgroups, and so is a plane at each end of a
 // chunk.  256 x 128 x 128 (8 rows of 128 nodes, 6 stored; 24 planes a chunk):
-// 1.7 first steps a node.  It is bound by vector instructions then, about
-// 550 a node and step of 64 lanes, 59 of 70 us.
+// 1.45 first steps a node.  It is bound by vector instructions then: 467 a
+// step of 64 nodes, whose issue takes 50 of the 70 us; the rest is waiting at
+// the planes' barriers and 94 % of the CUs at work.
 //
 // Per step, one at a time against this, sphere channels: FP32 256 x 128 x
 // 128 108.6 -> 69.9 us, 128^3 56.3 -> 38.4, 100^3 28.5 -> 20.6, 200^3 211 ->
@@ -56,10 +57,12 @@ constexpr uint32_t kMarchSlots = 256;  // one workgroup a CU
 // The cheapest cut of a lattice, and its cost: threads' plane steps per node
 // (a node on its own would cost 1).  A plane's rim rows and ends count, the
 // three planes by which a chunk's march is longer than its output, and the
-// last round of workgroups, which may be nearly empty.  Rows cut into strips
-// start anywhere in a cache line: 1.15 times as dear, 1.4 times where whole
-// rows are whole tiles (256 x 128 x 128 FP32, 1 strip 70 us, 2 strips of 66
-// threads 86; 121 x 67 x 93 FP64 31 and 29; 200^3 FP32 165 and 155).
+// last round of workgroups, which may be nearly empty.  Strips have
+// short rows that start anywhere in a cache line: a thread's step is 1.4
+// times as dear (200^3 FP32, 1 strip 165 us at a cost of 2.1, 2 strips 155 at
+// 1.4; 256 x 128 x 128 FP64 150 at 2.1, 4 strips 151 at 1.44), for FP64 with
+// rows that are no whole tiles either 1.15 times (121 x 67 x 93, 31 us at 2.4
+// and 4 strips 28 at 1.9).
 inline MarchPlan march_plan(const Grid& g, size_t bytes, double* cost) {
   const uint32_t threads = (uint32_t)march_threads(bytes);
   MarchPlan best{};
@@ -74,7 +77,7 @@ inline MarchPlan march_plan(const Grid& g, size_t bytes, double* cost) {
     if (p.rows < 3) continue;
     p.bands = (g.ny + p.rows - 3) / (p.rows - 2);
     const uint64_t columns = (uint64_t)p.strips * p.bands;
-    const double dear = strips == 1 ? 1.0 : g.nz % kTile == 0 ? 1.4 : 1.15;
+    const double dear = strips == 1 ? 1.0 : bytes == 4 || g.nz % kTile == 0 ? 1.4 : 1.15;
     // as many chunks as fill whole rounds of workgroups
     for (uint64_t rounds = 1; rounds <= 64; ++rounds) {
       uint64_t chunks = rounds * kMarchSlots / columns;
@@ -99,7 +102,8 @@ inline MarchPlan march_plan(const Grid& g, size_t bytes, double* cost) {
 // cost of 1 is about 9.5 ps a node FP32 and 17 FP64, a single step 26-30 and
 // 50-54, the more the smaller the lattice.
 constexpr uint32_t kMarchMinNodes = 350000, kMarchLargeNodes = 2000000;
-inline bool march_pays(const Grid& g, double cost) {
+inline bool march_pays(const Grid& g, size_t bytes, double cost) {
+  if (population_elems(19, g.n) * bytes >> 32) return false;  // 32-bit byte offsets
   return cost <= (g.n < kMarchLargeNodes ? 3.1 : 2.6);
 }
 
@@ -158,11 +162,13 @@ __device__ __forceinline__ void march_unit(const Grid& g, const MarchPlan& pl,
   y = fold(y, ny, g.flags & kWrapY);
   z = fold(z, nz, g.flags & kWrapZ);
   const uint32_t plane = g.ny * g.nz;
-  // the column's source columns, wrapped along each axis
-  const uint32_t cy[3] = {(uint32_t)(y + 1 == ny ? 0 : y + 1) * g.nz, (uint32_t)y * g.nz,
-                          (uint32_t)(y == 0 ? ny - 1 : y - 1) * g.nz};
-  const uint32_t cz[3] = {(uint32_t)(z + 1 == nz ? 0 : z + 1), (uint32_t)z,
-                          (uint32_t)(z == 0 ? nz - 1 : z - 1)};
+  // the column's source columns in bytes, wrapped along each axis
+  const uint32_t row = g.nz * (uint32_t)sizeof(T);
+  const uint32_t cy[3] = {(uint32_t)(y + 1 == ny ? 0 : y + 1) * row, (uint32_t)y * row,
+                          (uint32_t)(y == 0 ? ny - 1 : y - 1) * row};
+  const uint32_t cz[3] = {(uint32_t)(z + 1 == nz ? 0 : z + 1) * (uint32_t)sizeof(T),
+                          (uint32_t)z * (uint32_t)sizeof(T),
+                          (uint32_t)(z == 0 ? nz - 1 : z - 1) * (uint32_t)sizeof(T)};
   // LDS places of the neighbours: wrapped where a strip is a whole row, else
   // held inside (a rim's second step is not used)
   auto place = [&](int a, int b) {  // source of e_y = a, e_z = b
@@ -186,48 +192,70 @@ __device__ __forceinline__ void march_unit(const Grid& g, const MarchPlan& pl,
   const int xe = xs + (int)pl.planes < nx ? xs + (int)pl.planes : nx;
   auto fold_x = [&](int X) { return (uint32_t)fold(X, nx, wrap_x); };
   auto mask_of = [&](int X) {
-    return gload(mask + (fold_x(X) * plane + cy[1] + cz[1]));
+    return gload(mask + (fold_x(X) * plane + (cy[1] + cz[1]) / (uint32_t)sizeof(T)));
+  };
+  // Populations in byte offsets (below 2^32: march_pays) through a buffer
+  // resource: element (n, i) lies at v + v / kRow (Q - 1) kRow + i kRow, v
+  // being n in bytes, so a pulled address takes an add, a shift and one 24-bit
+  // multiply-add, and a bounced one two more (its part of i kRow that both
+  // share is the load's constant): 114 instructions a node instead of the 193
+  // of 64-bit addresses from element indices.
+  constexpr uint32_t kRow = kTile * (uint32_t)sizeof(T);
+  const auto from = buffer_rsrc(A, (g.n + kTile - 1) / kTile * (Q * kRow));
+  auto load = [&](uint32_t at, uint32_t shift) -> T {
+    const int off = (int)(at + shift % 4096u), rest = (int)(shift / 4096u * 4096u);
+    if constexpr (sizeof(T) == 4)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(from, off, rest, 0));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(from, off, rest, 0));
   };
   auto gather = [&](int X, uint32_t m, MarchLoad<T>& ld) {
+    constexpr uint32_t kSize = (uint32_t)sizeof(T);
     const uint32_t x0 = fold_x(X);
-    const uint32_t bx[3] = {(x0 + 1 == g.nx ? 0u : x0 + 1) * plane, x0 * plane,
-                            (x0 == 0 ? g.nx - 1 : x0 - 1) * plane};
+    const uint32_t bx[3] = {(x0 + 1 == g.nx ? 0u : x0 + 1) * plane * kSize, x0 * plane * kSize,
+                            (x0 == 0 ? g.nx - 1 : x0 - 1) * plane * kSize};
+    auto pull = [&](int i) {
+      const uint32_t v = bx[L::E[i][0] + 1] + cy[L::E[i][1] + 1] + cz[L::E[i][2] + 1];
+      return __umul24(v / kRow, (Q - 1) * kRow) + v;
+    };
     ld.m = m;
-    ld.own = pidx<Q>(bx[1] + cy[1] + cz[1], 0);
+    const uint32_t own = pull(0);
+    ld.own = own / kSize;
     if (__any((m & ((1u << Q) - 2u)) != 0u)) {
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
-        const uint32_t from =
-            pidx<Q>(bx[L::E[i][0] + 1] + cy[L::E[i][1] + 1] + cz[L::E[i][2] + 1], i);
-        const uint32_t back = ld.own + (uint32_t)L::INV[i] * kTile;
-        ld.raw[i] = gload(elem(A, i ? select_bit(m, i, back, from) : from));
+        const uint32_t lo = (uint32_t)(i < L::INV[i] ? i : L::INV[i]) * kRow;
+        const uint32_t a = pull(i) + ((uint32_t)i * kRow - lo);
+        const uint32_t b = own + ((uint32_t)L::INV[i] * kRow - lo);
+        ld.raw[i] = load(i ? select_bit(m, i, b, a) : a, lo);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < Q; ++i)
-        ld.raw[i] = gload(
-            elem(A, pidx<Q>(bx[L::E[i][0] + 1] + cy[L::E[i][1] + 1] + cz[L::E[i][2] + 1], i)));
+      for (int i = 0; i < Q; ++i) ld.raw[i] = load(pull(i), (uint32_t)i * kRow);
     }
   };
   const bool any_out = __any(out);
-  // row X - 1 as far as it is known: pulled along the plane and from X - 2;
-  // un: what row X pulls from X - 1; o: row X - 1's own e_x = +1 values
+  // plane X - 1 as far as it is known: pulled along it and from X - 2; un:
+  // what plane X pulls from X - 1; o: plane X - 1's own e_x = +1 values
   C r[Q], un[Q], o[Q];
   uint32_t mr = 0, ownr = 0;
 #pragma unroll
   for (int i = 0; i < Q; ++i) r[i] = un[i] = o[i] = (C)0;
-  MarchLoad<T> ld;
   uint32_t mnext = mask_of(xs);
+  MarchLoad<T> ld;
   gather(xs - 1, mask_of(xs - 1), ld);
+  // (two planes a turn, without copies of the loads in flight, spill
+  // registers: 256 x 128 x 128 FP32 105 us)
   for (int X = xs - 1; X <= xe; ++X) {
-    // the first step of row X
+    // plane X's first step (what solid nodes get is not read: the links to them
+    // bounce)
     C gv[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i) gv[i] = St::cvt_u(ld.raw[i]);
     const uint32_t m = ld.m & ~LBM_MASK_SOLID, own = ld.own;
     const bool solid = (ld.m & LBM_MASK_SOLID) != 0u;
     T f1[Q];
-    std_collide_node<Q, S, LID>(p, gv, m, solid, [&](auto fd, int i, auto v) {
+    std_collide_node<Q, S, LID, 2, 0>(p, gv, m, false, [&](auto fd, int i, auto v) {
       if constexpr (decltype(fd)::value)
         f1[i] = St::round_sr_u(v, sr_key(St::kShifted ? sr_node_hash(own) : 0u, i));
       else
@@ -238,7 +266,7 @@ __device__ __forceinline__ void march_unit(const Grid& g, const MarchPlan& pl,
 #pragma unroll
       for (int i = 1; i < Q; ++i) buf[i - 1][t] = f1[i];
     }
-    // the next row's loads run under the second step
+    // the next plane's loads run under the second step
     if (X < xe) {
       const uint32_t m1 = mnext;
       mnext = mask_of(X + 2);
@@ -246,14 +274,14 @@ __device__ __forceinline__ void march_unit(const Grid& g, const MarchPlan& pl,
     }
     __syncthreads();
     if (any_out) {
-      // row X - 1: what comes from row X
+      // plane X - 1: what comes from plane X
       if (X > xs) {
         C h[Q];
 #pragma unroll
         for (int i = 0; i < Q; ++i) {
           if (L::E[i][0] < 0) {
             const C v = St::cvt_u(buf[i - 1][nb(i)]);
-            h[i] = ((mr >> i) & 1u) ? o[L::INV[i]] : v;
+            h[i] = pick(mr, i, o[L::INV[i]], v);
           } else {
             h[i] = r[i];
           }
@@ -275,7 +303,7 @@ __device__ __forceinline__ void march_unit(const Grid& g, const MarchPlan& pl,
           }
         });
       }
-      // row X
+      // plane X
       const uint32_t mx = solid ? m | LBM_MASK_SOLID : m;
 #pragma unroll
       for (int i = 0; i < Q; ++i) {
@@ -283,9 +311,9 @@ __device__ __forceinline__ void march_unit(const Grid& g, const MarchPlan& pl,
           r[i] = St::cvt_u(f1[0]);
         } else if (L::E[i][0] == 0) {
           const C v = St::cvt_u(buf[i - 1][nb(i)]);
-          r[i] = ((mx >> i) & 1u) ? St::cvt_u(f1[L::INV[i]]) : v;
+          r[i] = pick(mx, i, St::cvt_u(f1[L::INV[i]]), v);
         } else if (L::E[i][0] > 0) {
-          r[i] = ((mx >> i) & 1u) ? St::cvt_u(f1[L::INV[i]]) : un[i];
+          r[i] = pick(mx, i, St::cvt_u(f1[L::INV[i]]), un[i]);
           un[i] = St::cvt_u(buf[i - 1][nb(i)]);
           o[i] = St::cvt_u(f1[i]);
         }

@@ -109,6 +109,16 @@ __device__ __forceinline__ uint32_t select_bit(uint32_t m, int i, uint32_t b, ui
   return r;
 }
 
+// the same for a value
+template <class C>
+__device__ __forceinline__ C pick(uint32_t m, int i, C b, C a) {
+  if constexpr (sizeof(C) == 4)
+    return __builtin_bit_cast(
+        C, select_bit(m, i, __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a)));
+  else
+    return ((m >> i) & 1u) ? b : a;
+}
+
 // Phase 1: issue every load of node n (no value is used here, so the loads
 // of several nodes can be in flight together).
 template <int Q, int S>

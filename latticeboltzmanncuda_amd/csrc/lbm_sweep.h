@@ -163,16 +163,6 @@ __device__ __forceinline__ C lane_down(C v) {
   }
 }
 
-// b where bit i of m is set, else a
-template <class C>
-__device__ __forceinline__ C pick(uint32_t m, int i, C b, C a) {
-  if constexpr (sizeof(C) == 4)
-    return __builtin_bit_cast(
-        C, select_bit(m, i, __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a)));
-  else
-    return ((m >> i) & 1u) ? b : a;
-}
-
 // What stage s keeps of its input: row X (the newest one) as far as it
 // enters row X's own update.  Directions in the order of Lat<9>: e_x = -1:
 // 1, 5, 6; e_x = 0: 0, 2, 3; e_x = +1: 4, 7, 8.
