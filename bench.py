@@ -96,7 +96,9 @@ def batched_section(steps, launch=None, chunk=100):
     """512 D2Q9 cavity/channel lattices (seed 4): plain per-lattice
     launches vs one persistent launch per step, replayed in hipGraph chunks
     of `chunk` steps (0: launched one by one), FP32 and FP16 storage; FP16
-    velocity error against FP64 storage."""
+    velocity error against FP64 storage.  The hbm_frac values count every
+    population read and written once a step, which a pass of several steps
+    does not do: they may exceed 1."""
     from latticeboltzmanncuda_amd import capi, workloads
     out = {"workload": "512 D2Q9 lattices (seed 4), sides log-uniform "
                        "32-512, cavity/channel, Re 100-1000, tau >= 0.51, "
@@ -187,8 +189,10 @@ def c4kernel_section(steps, launch=None):
 def lattice2d_section(steps):
     """One D2Q9 FP16 lattice of 4096^2 nodes (two population copies of
     604 MB, streamed from HBM): lid-driven cavity and body-force channel
-    with 10 % squares, run by the group step (two nodes per thread, chosen
-    for lattices this size) and, for comparison, by the one-node step."""
+    with 10 % squares, by the way chosen for lattices this size (several
+    steps in one pass; key "group") and, for comparison, by the one-node
+    step.  hbm_frac_36B counts every population read and written once a step,
+    which a pass of several steps does not do: it may exceed 1."""
     from latticeboltzmanncuda_amd import capi, workloads
     n = 4096
     sq = workloads.random_squares(n, n, 0.1, np.random.default_rng(7))
@@ -413,7 +417,7 @@ def reference_cpu_baseline(O, seconds, threads):
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles",
-                            "k_std_step_d3q19_f32_channel_traffic.json")
+                            "k_std_march_d3q19_f32_channel_traffic.json")
 
 
 def measured_traffic():
@@ -458,11 +462,12 @@ def main():
         raise RuntimeError("non-finite state after the timed steps")
     ms_per_step = ms / args.steps
     mlups = n * args.steps / (ms / 1e3) / 1e6
-    # the step reads and writes all 19 FP32 populations of every node (solid
-    # nodes included: their lanes store the rest state so that every store
-    # writes whole cache lines)
+    # a launch reads and writes all 19 FP32 populations of every node once
+    # (solid nodes included: their lanes store the rest state so that every
+    # store writes whole cache lines) and takes two steps with them
     bytes_per_launch = n * 2 * 19 * 4
-    achieved = bytes_per_launch / (ms_per_step / 1e3) / 1e9
+    steps_per_launch = 2
+    achieved = bytes_per_launch / (steps_per_launch * ms_per_step / 1e3) / 1e9
     out = {
         "metric": METRIC,
         "value": round(mlups, 1),
@@ -495,8 +500,9 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": measured_traffic(),
-            "kernel": "k_std_step<19, f32>",
+            "kernel": "k_std_march<f32>",
             "bytes_per_launch": bytes_per_launch,
+            "steps_per_launch": steps_per_launch,
             "copy_gbs": round(copy_gbs, 1),
             "frac_of_copy": round(achieved / copy_gbs, 4),
         },
