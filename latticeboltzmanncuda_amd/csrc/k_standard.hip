@@ -110,31 +110,11 @@ __global__ void __launch_bounds__(march_threads(sizeof(typename Store<S>::T)))
 // 4.8 / 5.6.
 constexpr uint32_t kEarlyNodes = 36000;
 
-// The step constants as a kernel's argument, or where k_put_coef left them:
-// many steps of a small lattice are bound by the host, which writes every
-// launch's arguments (32^3 FP32, 1000 steps: 4.1 us a launch with 0.5 KB of
-// them, 2.5 with a pointer; the step on the GPU 3.5).
-template <int S>
-struct CoefValue {
-  Coef<S> k;
-  __device__ const Coef<S>& get() const { return k; }
-};
-template <int S>
-struct CoefPointer {
-  const Coef<S>* k;
-  __device__ const Coef<S>& get() const { return *k; }
-};
-template <int S>
-__global__ void __launch_bounds__(64) k_put_coef(Coef<S> k, Coef<S>* out) {
-  if (threadIdx.x == 0) *out = k;
-}
-
-template <int Q, int S, class Args>
-__global__ void __launch_bounds__(64)
-    k_std_early(Grid g, const typename Store<S>::T* __restrict__ A,
-                typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
-                Args args) {
-  const Coef<S>& p = args.get();
+template <int Q, int S>
+__device__ __forceinline__ void early_unit(const Grid& g,
+                                           const typename Store<S>::T* __restrict__ A,
+                                           typename Store<S>::T* __restrict__ B,
+                                           const uint32_t* __restrict__ mask, const Coef<S>& p) {
   const uint32_t n = blockIdx.x * 64 + threadIdx.x;
   if (n >= g.n) return;
   NodeLoad<Q, S> ld;
@@ -151,6 +131,33 @@ __global__ void __launch_bounds__(64)
     else
       gstore(out + i * kTile, round_out<S>(o));
   });
+}
+
+// The step constants as a kernel's argument, or where k_put_coef left them:
+// many steps of a small lattice are bound by the host, which writes every
+// launch's arguments (32^3 FP32, 1000 steps: 4.1 us a launch with 0.5 KB of
+// them, 2.5 with a pointer; the step on the GPU 3.5).
+template <int Q, int S>
+__global__ void __launch_bounds__(64)
+    k_std_early(Grid g, const typename Store<S>::T* __restrict__ A,
+                typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
+                Coef<S> p) {
+  early_unit<Q, S>(g, A, B, mask, p);
+}
+// (k is an argument of its own and __restrict__: the constants are then read
+// by scalar loads ahead of the stores.  Inside a struct of arguments they
+// were read again behind every store that might have changed them: D3Q27
+// FP32 with a force 28^3 7.6 us a step.)
+template <int Q, int S>
+__global__ void __launch_bounds__(64)
+    k_std_early_at(Grid g, const typename Store<S>::T* __restrict__ A,
+                   typename Store<S>::T* __restrict__ B, const uint32_t* __restrict__ mask,
+                   const Coef<S>* __restrict__ k) {
+  early_unit<Q, S>(g, A, B, mask, *k);
+}
+template <int S>
+__global__ void __launch_bounds__(64) k_put_coef(Coef<S> k, Coef<S>* out) {
+  if (threadIdx.x == 0) *out = k;
 }
 
 // Groups of NV nodes per thread (std_group_step).
@@ -537,14 +544,12 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
       using T = typename Store<Tag::S>::T;
       const dim3 grid((g.n + 63) / 64);
       if constexpr (Tag::Q != 9) {
-        using Value = CoefValue<Tag::S>;
-        using Pointer = CoefPointer<Tag::S>;
         if (coef)
-          hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S, Pointer>), grid, dim3(64), 0, s, g,
-                             (const T*)A, (T*)B, mask, Pointer{(const Coef<Tag::S>*)coef});
+          hipLaunchKernelGGL((k_std_early_at<Tag::Q, Tag::S>), grid, dim3(64), 0, s, g,
+                             (const T*)A, (T*)B, mask, (const Coef<Tag::S>*)coef);
         else
-          hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S, Value>), grid, dim3(64), 0, s, g,
-                             (const T*)A, (T*)B, mask, Value{coef_of<Tag::S>(p)});
+          hipLaunchKernelGGL((k_std_early<Tag::Q, Tag::S>), grid, dim3(64), 0, s, g,
+                             (const T*)A, (T*)B, mask, coef_of<Tag::S>(p));
       }
     });
     if (drc) return drc;

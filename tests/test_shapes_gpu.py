@@ -14,6 +14,7 @@ must still be right, and waves with and without solid nodes take
 different code)."""
 import os
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -209,3 +210,31 @@ def test_small_3d_constants_are_those_of_the_call():
                     c.step(k)
             got.append(c.populations())
     assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("q", [19, 27])
+@pytest.mark.parametrize("storage", [capi.STORE_F32, capi.STORE_F64])
+def test_small_3d_constants_in_memory_cost_no_more(q, storage):
+    # the step is the same whether its constants are the launch's argument
+    # (calls of 15 steps) or lie in device memory (one call of 1200): reading
+    # them again behind the stores made it 1.4 to 1.6 times as long
+    print(f"case: D3Q{q} storage {storage}, constants in device memory",
+          flush=True)
+    n = 24
+    cfg = capi.make_config(n, n, n, lattice=q, storage=storage, tau=0.7,
+                           periodic=(1, 0, 0), force=(1e-6, 0, 0))
+    best = {}
+    with capi.Context(cfg) as c:
+        c.init_equilibrium()
+        for _ in range(6):
+            for calls in (80, 1):
+                c.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(calls):
+                    c.step(1200 // calls)
+                c.synchronize()
+                dt = time.perf_counter() - t0
+                best[calls] = min(best.get(calls, dt), dt)
+    print(f"  argument {best[80] / 1.2e-3:.2f} us a step, memory "
+          f"{best[1] / 1.2e-3:.2f}", flush=True)
+    assert best[1] < 1.2 * best[80]
