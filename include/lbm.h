@@ -218,6 +218,22 @@ int lbm_get_force(lbm_ctx* ctx, float out[3]);
  * Reference mode: Lattice::simulateLattice (Lattice.cpp:222-226), stream
  * then collide. */
 int lbm_step(lbm_ctx* ctx, int n);
+/* The launches of lbm_step(ctx, n) on a standard-mode lattice of this
+ * configuration (with LBM_GROUP_STEP as it is set): launches[k - 1] of them
+ * take k steps each; *kernel takes those of several steps or, where there
+ * are none, the single ones.  A host computation: no GPU call (no
+ * counterpart in the reference). */
+#define LBM_MAX_LAUNCH_STEPS 8
+enum lbm_step_kernel {
+  LBM_STEP_NODE = 0,  /* one step, one node per thread                  */
+  LBM_STEP_GROUP = 1, /* one step, 2 or 4 nodes per thread (D2Q9 16-bit) */
+  LBM_STEP_EARLY = 2, /* one step of a small 3-D lattice                 */
+  LBM_STEP_BOX = 3,   /* 2 to 4 or 8 steps of a small D2Q9 lattice       */
+  LBM_STEP_SWEEP = 4, /* 2 to 4 steps of a large D2Q9 lattice            */
+  LBM_STEP_MARCH = 5  /* 2 steps of a large D3Q19 lattice                */
+};
+int lbm_step_route(const lbm_config* cfg, int n, int* kernel,
+                   int32_t launches[LBM_MAX_LAUNCH_STEPS]);
 /* n steps of each of count standard-mode lattices, one lbm_step launch
  * per lattice per step (the unbatched way to step many lattices; no
  * counterpart in the reference). */

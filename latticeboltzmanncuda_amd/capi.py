@@ -27,6 +27,8 @@ ERR_INVALID, ERR_BUDGET, ERR_UNSTABLE = 1, 6, 8
 # serving request status
 SERVE_CONVERGED, SERVE_STEP_LIMIT, SERVE_REJECTED, SERVE_DIVERGED, \
     SERVE_UNSTABLE = 0, 1, 2, 3, 4
+# kernels of lbm_step (step_route)
+STEP_NODE, STEP_GROUP, STEP_EARLY, STEP_BOX, STEP_SWEEP, STEP_MARCH = range(6)
 FLOW_NONE, FLOW_POINT, FLOW_PLANE, FLOW_BOX, FLOW_MASK = 0, 1, 2, 3, 4
 FLAG_INTERNAL, FLAG_REFLECTED = 1, 2
 MASK_SOLID = 1 << 31
@@ -162,6 +164,8 @@ _SIGNATURES = {
     "lbm_set_force": (C.c_int, [CTX, P]),
     "lbm_get_force": (C.c_int, [CTX, P]),
     "lbm_step": (C.c_int, [CTX, C.c_int]),
+    "lbm_step_route": (C.c_int, [C.POINTER(Config), C.c_int,
+                                 C.POINTER(C.c_int), C.POINTER(i32)]),
     "lbm_step_each": (C.c_int, [P, i32, C.c_int]),
     "lbm_step_reference": (C.c_int, [CTX, C.c_int, C.c_int]),
     "lbm_time_steps": (C.c_int, [CTX, C.c_int, C.POINTER(C.c_float)]),
@@ -610,6 +614,18 @@ def cell_reynolds(cfg: Config) -> float:
     if v < 0:
         check(int(-v), "lbm_cell_reynolds")
     return float(v)
+
+
+def step_route(cfg: Config, n: int) -> tuple[int, dict[int, int]]:
+    """The launches of step(n) on a lattice of this configuration: the kernel
+    (STEP_*) of those that take several steps, or of the single ones where
+    there are none, and {steps of a launch: launches} (lbm_step_route; no GPU
+    call)."""
+    kernel = C.c_int(0)
+    launches = (i32 * 8)()
+    check(load().lbm_step_route(C.byref(cfg), n, C.byref(kernel), launches),
+          "lbm_step_route")
+    return kernel.value, {k + 1: v for k, v in enumerate(launches) if v}
 
 
 def step_each(contexts, n: int) -> None:

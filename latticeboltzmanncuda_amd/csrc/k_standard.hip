@@ -498,12 +498,23 @@ int launch_put_coef(int q, int storage, const StdParams& p, void* coef, hipStrea
   return LBM_OK;
 }
 
+namespace {
+bool streams(int q, int storage, const Grid& g) {
+  return streaming_stores(2 * population_elems(q, g.n) * storage_bytes(storage));
+}
+}  // namespace
+
+int std_single_kernel(int q, int storage, const Grid& g) {
+  if (group_step_width(q, storage, g, streams(q, storage, g))) return LBM_STEP_GROUP;
+  return q != 9 && g.n <= kEarlyNodes ? LBM_STEP_EARLY : LBM_STEP_NODE;
+}
+
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
                     const uint32_t* mask, const uint32_t* cls,
                     const StdParams& p, int rev, hipStream_t s, const void* coef) {
   const unsigned nb = blocks_for(g.n);
   const bool lid = p.lid_axis >= 0;
-  const bool nt = streaming_stores(2 * population_elems(q, g.n) * storage_bytes(storage));
+  const bool nt = streams(q, storage, g);
   // measured on MI355X: with streaming stores, alternating the tile order
   // between steps is fastest; without them, a fixed order is
   const int r = nt ? rev : 0;
@@ -538,7 +549,7 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
     LBM_HIP(hipGetLastError());
     return LBM_OK;
   }
-  if (q != 9 && g.n <= kEarlyNodes) {
+  if (std_single_kernel(q, storage, g) == LBM_STEP_EARLY) {
     const int drc = dispatch_qs(q, storage, [&](auto tag) {
       using Tag = decltype(tag);
       using T = typename Store<Tag::S>::T;
@@ -615,8 +626,7 @@ bool std_sweeps(int q, int storage, const Grid& g) {
   if (q != 9 || single_steps()) return false;
   // 16-bit lattices that fit the Infinity Cache are as fast one step at a
   // time (2900 x 1700: 24.2-30.5 against 24.7-28.9 us), larger ones are not
-  return storage_bytes(storage) == 2 ? streaming_stores(2 * population_elems(q, g.n) * 2)
-                                     : g.n >= kSweepMinNodes;
+  return storage_bytes(storage) == 2 ? streams(q, storage, g) : g.n >= kSweepMinNodes;
 }
 
 int launch_std_sweep(int k, int storage, const Grid& g, const SweepPlan& pl, const void* A,

@@ -286,6 +286,18 @@ int validate_config(const lbm_config* cfg) {
   return LBM_OK;
 }
 
+Grid make_grid(const lbm_config& cfg) {
+  Grid g{};
+  g.nx = (uint32_t)cfg.nx;
+  g.ny = (uint32_t)cfg.ny;
+  g.nz = (uint32_t)cfg.nz;
+  g.n = g.nx * g.ny * g.nz;
+  g.dz = make_magic(g.nz);
+  g.dy = make_magic(g.ny);
+  g.flags = wrap_bits(cfg.periodic);
+  return g;
+}
+
 // The geometry tables, rebuilt after a change of flags or records.
 int rebuild_special(lbm_ctx* c) {
   if (!c->special_dirty) return LBM_OK;
@@ -298,23 +310,54 @@ int rebuild_special(lbm_ctx* c) {
 // 1 us of host time each against 3 to 4 us).
 constexpr int kPutSteps = 16;
 
+// How a call of n steps of a lattice is launched: `kernel` (lbm_step_kernel)
+// takes the launches of several steps or, where there are none, the single
+// ones; launches[k]: how many take k steps each, the long ones first.
+struct StepPlan {
+  int kernel = LBM_STEP_NODE;
+  int launches[LBM_MAX_LAUNCH_STEPS + 1] = {};
+  MarchPlan march{};
+  SweepPlan sweep{};
+};
+
+// As many launches, odd or even, as there are steps: a caller who captures
+// them finds the state in the same buffer as after single steps.
+StepPlan plan_steps(int q, int storage, const Grid& g, int n) {
+  StepPlan p;
+  if (n <= 1) {
+    p.kernel = std_single_kernel(q, storage, g);
+    p.launches[1] = n;
+    return p;
+  }
+  const int box = std_box_steps(q, storage, g);
+  int rest = n;  // taken as evenly as can be
+  if (box || std_sweeps(q, storage, g)) {
+    p.kernel = box ? LBM_STEP_BOX : LBM_STEP_SWEEP;
+    // boxes of 8 steps come in pairs
+    if (box == 8) p.launches[8] = n / 16 * 2;
+    rest -= 8 * p.launches[8];
+    for (int passes = sweep_passes(rest); passes > 0; --passes) {
+      const int k = (rest + passes - 1) / passes;
+      ++p.launches[k];
+      rest -= k;
+    }
+    if (!box)
+      p.sweep = sweep_plan(g, sweep_chunk_rows(1, [&](size_t) -> const Grid& { return g; }, storage));
+  } else if (n >= 4 && std_marches(q, storage, g, &p.march)) {
+    p.kernel = LBM_STEP_MARCH;
+    p.launches[2] = n / 4 * 2;
+    p.launches[1] = n % 4;
+  } else {
+    p.launches[1] = n;
+  }
+  if (p.launches[1] == n) p.kernel = std_single_kernel(q, storage, g);
+  return p;
+}
+
 int step_standard(lbm_ctx* c, int n) {
   const StdParams p = make_std_params(c->cfg);
   const int storage = device_storage(c->cfg.mode, c->cfg.storage);
-  const int box = n > 1 ? std_box_steps(c->q, storage, c->grid) : 0;
-  const bool sweeps = n > 1 && !box && std_sweeps(c->q, storage, c->grid);
-  const SweepPlan plan =
-      sweeps ? sweep_plan(c->grid, sweep_chunk_rows(
-                                       1, [&](size_t) -> const Grid& { return c->grid; }, storage))
-             : SweepPlan{};
-  // As many passes, odd or even, as there are steps: a caller who captures
-  // the launches finds the state in the same buffer as after single steps.
-  // Boxes of 8 steps come in pairs, the rest is spread like a sweep's.
-  // So do the marches of two.
-  MarchPlan march{};
-  const int pairs = n >= 4 && std_marches(c->q, storage, c->grid, &march) ? n / 4 * 2 : 0;
-  const int eights = box == 8 ? n / 16 * 2 : 0;
-  const int passes = pairs ? n - pairs : eights + (sweeps || box ? sweep_passes(n - 8 * eights) : n);
+  const StepPlan plan = plan_steps(c->q, storage, c->grid, n);
   // the constants as they are now, for this call's launches alone: whoever
   // changes them, or captures the call, finds what a launch with them as
   // arguments would do
@@ -323,23 +366,24 @@ int step_standard(lbm_ctx* c, int n) {
     if (int rc = launch_put_coef(c->q, storage, p, c->coef, c->stream)) return rc;
     coef = c->coef;
   }
-  for (int s = 0, left = n; s < passes; ++s) {
-    const int k = s < pairs ? 2 : s < eights ? 8 : (left + (passes - s) - 1) / (passes - s);
-    int rc = s < pairs
-                 ? launch_std_march(storage, c->grid, march, c->f[c->cur], c->f[c->cur ^ 1],
-                                    c->mask, p, c->stream)
-             : k > 1 && box
-                 ? launch_std_box(k, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1], c->mask,
-                                  c->cls, p, c->stream)
-             : k > 1 ? launch_std_sweep(k, storage, c->grid, plan, c->f[c->cur], c->f[c->cur ^ 1],
-                                      c->mask, p, c->stream)
-                   : launch_std_step(c->q, storage, c->grid, c->f[c->cur], c->f[c->cur ^ 1],
-                                     c->mask, c->cls, p, (int)(c->steps_done & 1), c->stream, coef);
-    if (rc) return rc;
-    c->cur ^= 1;
-    c->steps_done += k;
-    left -= k;
-  }
+  for (int k = LBM_MAX_LAUNCH_STEPS; k > 0; --k)
+    for (int s = 0; s < plan.launches[k]; ++s) {
+      const void* A = c->f[c->cur];
+      void* B = c->f[c->cur ^ 1];
+      int rc;
+      if (k == 1)
+        rc = launch_std_step(c->q, storage, c->grid, A, B, c->mask, c->cls, p,
+                             (int)(c->steps_done & 1), c->stream, coef);
+      else if (plan.kernel == LBM_STEP_MARCH)
+        rc = launch_std_march(storage, c->grid, plan.march, A, B, c->mask, p, c->stream);
+      else if (plan.kernel == LBM_STEP_BOX)
+        rc = launch_std_box(k, storage, c->grid, A, B, c->mask, c->cls, p, c->stream);
+      else
+        rc = launch_std_sweep(k, storage, c->grid, plan.sweep, A, B, c->mask, p, c->stream);
+      if (rc) return rc;
+      c->cur ^= 1;
+      c->steps_done += k;
+    }
   return LBM_OK;
 }
 
@@ -462,14 +506,8 @@ int lbm_create(const lbm_config* cfg, void* stream, lbm_ctx** out) {
   c->cfg = *cfg;
   c->q = cfg->lattice;
   c->elem = storage_bytes(cfg->storage);
-  Grid& g = c->grid;
-  g.nx = (uint32_t)cfg->nx;
-  g.ny = (uint32_t)cfg->ny;
-  g.nz = (uint32_t)cfg->nz;
-  g.n = g.nx * g.ny * g.nz;
-  g.dz = make_magic(g.nz);
-  g.dy = make_magic(g.ny);
-  g.flags = wrap_bits(cfg->periodic);
+  c->grid = make_grid(*cfg);
+  const Grid& g = c->grid;
   c->flow.kind = LBM_FLOW_NONE;
   auto bail = [&](int code) {
     lbm_destroy(c);
@@ -846,6 +884,20 @@ int lbm_step(lbm_ctx* c, int n) {
   TraceRange tr("lbm_step");
   return c->cfg.mode == LBM_MODE_STANDARD ? step_standard(c, n)
                                           : step_reference_fused(c, n);
+}
+
+int lbm_step_route(const lbm_config* cfg, int n, int* kernel,
+                   int32_t launches[LBM_MAX_LAUNCH_STEPS]) {
+  if (int rc = validate_config(cfg)) return rc;
+  if (cfg->mode != LBM_MODE_STANDARD)
+    return fail(LBM_ERR_STATE, "lbm_step_route needs a standard-mode configuration");
+  if (n < 0) return fail(LBM_ERR_INVALID, "negative step count");
+  if (!kernel || !launches) return fail(LBM_ERR_INVALID, "null output");
+  const StepPlan p =
+      plan_steps(cfg->lattice, device_storage(cfg->mode, cfg->storage), make_grid(*cfg), n);
+  *kernel = p.kernel;
+  for (int k = 1; k <= LBM_MAX_LAUNCH_STEPS; ++k) launches[k - 1] = p.launches[k];
+  return LBM_OK;
 }
 
 int lbm_step_each(lbm_ctx* const* ctxs, int32_t count, int n) {

@@ -43,6 +43,7 @@
   X(int, lbm_set_force, (lbm_ctx* a, const float b[3]), (a, b))                                \
   X(int, lbm_get_force, (lbm_ctx* a, float b[3]), (a, b))                                      \
   X(int, lbm_step, (lbm_ctx* a, int b), (a, b))                                                \
+  X(int, lbm_step_route, (const lbm_config* a, int b, int* c, int32_t d[8]), (a, b, c, d))     \
   X(int, lbm_step_each, (lbm_ctx* const* a, int32_t b, int c), (a, b, c))                      \
   X(int, lbm_step_reference, (lbm_ctx* a, int b, int c), (a, b, c))                            \
   X(int, lbm_time_steps, (lbm_ctx* a, int b, float* c), (a, b, c))                             \

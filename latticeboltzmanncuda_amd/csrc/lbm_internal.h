@@ -148,6 +148,8 @@ int api_exception() noexcept;
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
                     const uint32_t* mask, const uint32_t* cls,
                     const StdParams& p, int rev, hipStream_t s, const void* coef = nullptr);
+// The kernel that launch_std_step takes (lbm_step_kernel).
+int std_single_kernel(int q, int storage, const Grid& g);
 // Lattices whose steps can read their constants from device memory
 // (launch_std_step's coef), once launch_put_coef has written them there in
 // stream order: for calls of many steps, whose launches then carry less.

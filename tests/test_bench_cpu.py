@@ -59,3 +59,24 @@ def test_cpu_baseline_leg_runs(monkeypatch):
     ref = out["reference_main_loop"]
     assert ref["reflection_records"] > 0
     assert ref["all_threads"]["mlups"] > 0 and ref["single_thread"]["mlups"] > 0
+
+
+def test_bench_counts_the_launches_of_the_timed_call():
+    b = load_bench()
+    from latticeboltzmanncuda_amd import capi
+    cfg = capi.make_config(*b.DIMS, lattice=capi.D3Q19, tau=b.TAU,
+                           periodic=(1, 0, 0), force=b.FORCE)
+    nbytes = 256 * 128 * 128 * 2 * 19 * 4
+    for steps, launches, kernel in ((1, 1, "k_std_step"), (3, 3, "k_std_step"),
+                                    (4, 2, "k_std_march"),
+                                    (7, 5, "k_std_march"),
+                                    (20, 10, "k_std_march"),
+                                    (5000, 2500, "k_std_march")):
+        r = b.roofline(cfg, steps, 0.1 * steps)
+        assert r["kernel"] == kernel + "<f32>"
+        assert sum(r["launches_by_steps"].values()) == launches
+        assert sum(k * v for k, v in r["launches_by_steps"].items()) == steps
+        assert abs(r["steps_per_launch"] - steps / launches) < 1e-3
+        assert abs(r["achieved"] - nbytes * launches / (1e-4 * steps) / 1e9) \
+            < 0.1
+        assert (r["traffic"] is None) == (kernel == "k_std_step")

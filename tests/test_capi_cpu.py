@@ -159,3 +159,29 @@ def test_struct_mirrors_match_header(cls, cname, tmp_path):
     got = _c_layout(cname, fields, tmp_path)
     assert got[:-1] == [getattr(cls, f).offset for f in fields]
     assert got[-1] == C.sizeof(cls)
+
+
+def test_step_route_takes_every_step_once():
+    # every launch swaps the buffers, so their count is as odd or even as the
+    # steps'; the query needs no GPU
+    shapes = [(9, (64, 64, 1)), (9, (300, 330, 1)), (9, (900, 1200, 1)),
+              (9, (4096, 4096, 1)), (9, (100000, 20, 1)), (9, (1, 5, 1)),
+              (19, (32, 32, 32)), (19, (128, 128, 128)), (19, (200, 200, 200)),
+              (27, (20, 20, 20)), (27, (128, 128, 128))]
+    for q, dims in shapes:
+        for storage in range(4):
+            cfg = capi.make_config(*dims, lattice=q, storage=storage, tau=0.7)
+            for n in list(range(40)) + [1000, 5003]:
+                kernel, by = capi.step_route(cfg, n)
+                assert sum(k * v for k, v in by.items()) == n
+                assert sum(by.values()) % 2 == n % 2
+                several = any(k > 1 for k in by)
+                assert several == (kernel in (capi.STEP_BOX, capi.STEP_SWEEP,
+                                              capi.STEP_MARCH))
+    with pytest.raises(capi.LbmError):
+        capi.step_route(capi.make_config(4, 4, 4), -1)
+    with pytest.raises(capi.LbmError):
+        capi.step_route(capi.make_config(0, 4, 4), 1)
+    with pytest.raises(capi.LbmError):
+        capi.step_route(capi.make_config(4, 4, 4, lattice=27,
+                                         mode=capi.MODE_REFERENCE), 1)
