@@ -103,12 +103,30 @@ __global__ void __launch_bounds__(march_threads(sizeof(typename Store<S>::T)))
 }
 
 // Small 3-D lattices (std_gather_early), one wavefront per workgroup: they
-// have fewer of them than would fill the GPU.  Up to kEarlyNodes, where
-// twice the loads cost less than the latencies: per step, loads in turn
-// against early, D3Q19 24^3 FP32 3.8 -> 3.6 us, 32^3 FP32 3.9 -> 3.5, FP64
-// 5.0 -> 4.2, D3Q27 32^3 FP32 5.0 -> 4.2, FP64 6.3 -> 5.3; 40^3 D3Q19 FP32
-// 4.8 / 5.6.
-constexpr uint32_t kEarlyNodes = 36000;
+// have fewer of them than would fill the GPU, so that twice the loads cost
+// less than the latencies they overlap.
+//
+// Where that ends, per step, loads in turn against early (cavity, forced
+// channel, periodic):
+//  - one workgroup a CU (16,384 nodes) gains 4-24 %: D3Q19 FP32 24^3 3.8 ->
+//    3.5 us, FP64 channel 5.1 -> 4.2; D3Q27 FP32 24^3 4.3 -> 4.1.  D3Q27 FP64
+//    only up to 12,288: 23^3 5.2 -> 5.0, 25^3 5.4 / 5.8;
+//  - above that the second read of a row costs more than the first saved
+//    (D3Q19 28^3 FP64 4.6 / 4.8, 33^3 FP32 4.1 / 4.5; D3Q27 FP64 28^3 5.9 /
+//    6.5), but not where planes are whole turns of the XCDs (512 nodes: eight
+//    workgroups), so that rows along x come from the XCD's own L2: 32^3
+//    D3Q19 FP32 3.9 -> 3.5, FP64 4.9 -> 4.2, D3Q27 FP32 4.8 -> 4.1, FP64 6.3
+//    -> 5.4;
+//  - D3Q19 with 16 bits moves half the bytes: 28^3 3.7 -> 3.5, 31^3 3.7-4.0
+//    -> 3.6-3.8, 33^3 3.7-4.0 / 3.8-4.1.
+constexpr uint32_t kEarlyNodes = 16384, kEarlyNodesD3Q27F64 = 12288, kEarlyMaxNodes = 32768;
+bool takes_early(int q, int storage, const Grid& g) {
+  if (q == 9 || g.n > kEarlyMaxNodes) return false;
+  const size_t bytes = storage_bytes(storage);
+  if (bytes == 2 && q == 19) return true;
+  return g.n <= (bytes == 8 && q == 27 ? kEarlyNodesD3Q27F64 : kEarlyNodes) ||
+         g.ny * g.nz % (8 * kTile) == 0;
+}
 
 template <int Q, int S>
 __device__ __forceinline__ void early_unit(const Grid& g,
@@ -485,7 +503,7 @@ int launch_std_march(int storage, const Grid& g, const MarchPlan& pl, const void
   return LBM_OK;
 }
 
-bool std_takes_coef(int q, const Grid& g) { return q != 9 && g.n <= kEarlyNodes; }
+bool std_takes_coef(int q, int storage, const Grid& g) { return takes_early(q, storage, g); }
 
 int launch_put_coef(int q, int storage, const StdParams& p, void* coef, hipStream_t s) {
   const int drc = dispatch_qs(q, storage, [&](auto tag) {
@@ -506,7 +524,7 @@ bool streams(int q, int storage, const Grid& g) {
 
 int std_single_kernel(int q, int storage, const Grid& g) {
   if (group_step_width(q, storage, g, streams(q, storage, g))) return LBM_STEP_GROUP;
-  return q != 9 && g.n <= kEarlyNodes ? LBM_STEP_EARLY : LBM_STEP_NODE;
+  return takes_early(q, storage, g) ? LBM_STEP_EARLY : LBM_STEP_NODE;
 }
 
 int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
@@ -549,7 +567,7 @@ int launch_std_step(int q, int storage, const Grid& g, const void* A, void* B,
     LBM_HIP(hipGetLastError());
     return LBM_OK;
   }
-  if (std_single_kernel(q, storage, g) == LBM_STEP_EARLY) {
+  if (takes_early(q, storage, g)) {
     const int drc = dispatch_qs(q, storage, [&](auto tag) {
       using Tag = decltype(tag);
       using T = typename Store<Tag::S>::T;

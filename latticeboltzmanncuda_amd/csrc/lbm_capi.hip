@@ -362,7 +362,7 @@ int step_standard(lbm_ctx* c, int n) {
   // changes them, or captures the call, finds what a launch with them as
   // arguments would do
   const void* coef = nullptr;
-  if (n >= kPutSteps && std_takes_coef(c->q, c->grid)) {
+  if (n >= kPutSteps && std_takes_coef(c->q, storage, c->grid)) {
     if (int rc = launch_put_coef(c->q, storage, p, c->coef, c->stream)) return rc;
     coef = c->coef;
   }

@@ -154,7 +154,7 @@ int std_single_kernel(int q, int storage, const Grid& g);
 // (launch_std_step's coef), once launch_put_coef has written them there in
 // stream order: for calls of many steps, whose launches then carry less.
 constexpr size_t kCoefBytes = 960;
-bool std_takes_coef(int q, const Grid& g);
+bool std_takes_coef(int q, int storage, const Grid& g);
 int launch_put_coef(int q, int storage, const StdParams& p, void* coef, hipStream_t s);
 // The most steps that one launch takes of a small D2Q9 lattice (8 or 4;
 // launch_std_box takes 8 or 2 to 4), 0 for the other lattices.

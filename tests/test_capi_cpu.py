@@ -185,3 +185,26 @@ def test_step_route_takes_every_step_once():
     with pytest.raises(capi.LbmError):
         capi.step_route(capi.make_config(4, 4, 4, lattice=27,
                                          mode=capi.MODE_REFERENCE), 1)
+
+
+def test_early_loads_only_where_they_are_faster():
+    # lattices on both sides of the rule, as measured (see k_standard.hip)
+    F32, F64, F16, BF16 = (capi.STORE_F32, capi.STORE_F64, capi.STORE_F16,
+                           capi.STORE_BF16)
+    early, node = capi.STEP_EARLY, capi.STEP_NODE
+    for q, storage, dims, want in (
+            (19, F32, (24, 24, 24), early), (19, F32, (32, 32, 32), early),
+            (19, F32, (64, 16, 16), early), (19, F32, (30, 30, 30), node),
+            (19, F32, (33, 33, 33), node), (19, F64, (25, 25, 25), early),
+            (19, F64, (28, 28, 28), node), (19, F64, (32, 32, 32), early),
+            (19, F64, (33, 33, 33), node), (19, F16, (31, 31, 31), early),
+            (19, BF16, (32, 32, 32), early), (19, F16, (33, 33, 33), node),
+            (27, F32, (24, 24, 24), early), (27, F32, (29, 29, 29), node),
+            (27, F32, (32, 32, 32), early), (27, F32, (24, 24, 48), node),
+            (27, F64, (23, 23, 23), early), (27, F64, (25, 25, 25), node),
+            (27, F64, (32, 32, 32), early), (27, F64, (33, 33, 33), node),
+            (27, F16, (24, 24, 24), early), (27, BF16, (30, 30, 30), node),
+            (27, F16, (33, 33, 33), node), (19, F32, (40, 32, 32), node)):
+        kernel, by = capi.step_route(
+            capi.make_config(*dims, lattice=q, storage=storage, tau=0.7), 100)
+        assert (kernel, by) == (want, {1: 100}), (q, storage, dims)

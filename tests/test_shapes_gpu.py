@@ -238,3 +238,35 @@ def test_small_3d_constants_in_memory_cost_no_more(q, storage):
     print(f"  argument {best[80] / 1.2e-3:.2f} us a step, memory "
           f"{best[1] / 1.2e-3:.2f}", flush=True)
     assert best[1] < 1.2 * best[80]
+
+
+# the edges of the rule that chooses early loads, from both sides
+EDGE_DIMS = [(16, 32, 32), (1, 1, 16385), (12288, 1, 1), (31, 27, 27),
+             (2, 32, 512), (31, 32, 33), (32, 32, 32), (8, 64, 64)]
+
+
+@pytest.mark.parametrize("q", [19, 27])
+@pytest.mark.parametrize("storage", [capi.STORE_F32, capi.STORE_F64,
+                                     capi.STORE_F16])
+def test_early_loads_at_their_limits_equal_batch(q, storage):
+    for k, dims in enumerate(EDGE_DIMS):
+        print(f"case: D3Q{q} {dims} storage {storage}, early limits",
+              flush=True)
+        rng = np.random.default_rng(40 + k)
+        n = dims[0] * dims[1] * dims[2]
+        per = ((1, 0, 0), (1, 1, 1), (0, 0, 1))[k % 3]
+        cfg = capi.make_config(*dims, lattice=q, storage=storage, tau=0.7,
+                               periodic=per, force=(1e-5, 0, 2e-6 * (k % 2)))
+        solid = (rng.random(n) < 0.15).astype(np.uint8)
+        got = []
+        with capi.Batch(storage) as b:
+            m = b.add(cfg, solid)
+            b.step(19)
+            got.append(m.populations(np.float64))
+        with capi.Context(cfg) as c:
+            c.upload_solid(solid)
+            c.init_equilibrium()
+            c.step(2)
+            c.step(17)
+            got.append(c.populations(np.float64))
+        assert np.array_equal(*got)
