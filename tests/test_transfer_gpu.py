@@ -3,8 +3,10 @@ up comes down unchanged, for sizes around the direct copy's limit, one chunk,
 the ring of slots and the threaded copies, from several threads at once, and
 the moments' two arrays (which share their chunks) equal the direct
 read-back's."""
+import ctypes
 import sys
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -84,3 +86,70 @@ def test_moments_pieces(dims):
         v3 = np.zeros(3 * n, np.float32)
         capi.check(c.lib.lbm_moments(c.h, None, v3.ctypes.data), "moments")
         assert np.array_equal(v2, v3)
+
+
+def hip():
+    """The HIP runtime that the library runs on."""
+    capi.load()
+    with open("/proc/self/maps") as fh:
+        path = next(l.split()[-1] for l in fh if "libamdhip64" in l)
+    return ctypes.CDLL(path)
+
+
+def flat(nbytes):
+    """A lattice whose moments fill so many bytes."""
+    return capi.make_config(1024, nbytes // 16 // 1024, 1, lattice=capi.D2Q9,
+                            tau=0.8, periodic=(1, 1, 0))
+
+
+@pytest.mark.parametrize("kind", ["pinned", "managed"])
+def test_memory_of_the_runtime_is_copied_directly(kind):
+    # a result (and an upload) in pinned memory takes as long as the runtime's
+    # own copy of it, not the detour through the library's pinned slots
+    say(f"case: {kind} host memory")
+    rt, nbytes = hip(), 256 << 20
+    p = ctypes.c_void_p()
+    size = ctypes.c_size_t(nbytes)
+    if kind == "pinned":
+        assert rt.hipHostMalloc(ctypes.byref(p), size, 0) == 0
+    else:
+        assert rt.hipMallocManaged(ctypes.byref(p), size, 1) == 0
+    try:
+        with capi.Context(flat(nbytes)) as c:
+            c.init_equilibrium(1.0 + 0.01 * np.random.default_rng(3).random(c.n))
+            c.step(2)
+            want = c.moments()
+            got = np.frombuffer((ctypes.c_float * (4 * c.n)).from_address(
+                p.value), np.float32)
+            got[:] = 0  # the CPU holds its pages
+            best = 1e9
+            for _ in range(4):
+                c.synchronize()
+                t0 = time.perf_counter()
+                capi.check(c.lib.lbm_moments(c.h, p, p.value + 4 * c.n),
+                           "moments")
+                best = min(best, time.perf_counter() - t0)
+            assert np.array_equal(got[:c.n], want[0])
+            assert np.array_equal(got[c.n:].reshape(3, -1), want[1])
+            if kind == "pinned":
+                d = ctypes.c_void_p()
+                assert rt.hipMalloc(ctypes.byref(d), size) == 0
+                direct = 1e9
+                for _ in range(4):
+                    t0 = time.perf_counter()
+                    assert rt.hipMemcpy(p, d, size, 2) == 0
+                    direct = min(direct, time.perf_counter() - t0)
+                rt.hipFree(d)
+                say(f"  moments {best * 1e3:.2f} ms, copy alone "
+                    f"{direct * 1e3:.2f}")
+                assert best < 1.35 * direct + 3e-4
+        f = np.frombuffer((ctypes.c_float * (nbytes // 4)).from_address(
+            p.value), np.float32)
+        n = nbytes // 108
+        f[:27 * n] = np.random.default_rng(4).random(27 * n, np.float32)
+        with capi.Context(capi.make_config(n, 1, 1, lattice=27,
+                                           mode=capi.MODE_REFERENCE)) as c:
+            capi.check(c.lib.lbm_set_populations_f32(c.h, p), "populations")
+            assert np.array_equal(c.populations(), f[:27 * n])
+    finally:
+        (rt.hipHostFree if kind == "pinned" else rt.hipFree)(p)
