@@ -22,6 +22,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -108,12 +110,60 @@ struct Ring {
   hipEvent_t event(size_t j) const { return r.ev[j % kSlots]; }
 };
 
+// What the threads of a copy wait for: chunks below `open` may be taken.
+// The first of them comes behind everything that the stream still has to do,
+// so a thread sleeps until then; afterwards its next chunk is a few DMAs of
+// 0.1 ms away, and a thread looks for that long before it sleeps (64 MiB 2.9
+// ms where it slept at once, 2.4 so).  Threads that only yielded kept six
+// CPUs busy for as long as the steps before a result took.
+class Gate {
+ public:
+  explicit Gate(size_t open) : open_(open) {}
+  // chunks below n are there
+  void raise(size_t n) {
+    {
+      std::lock_guard<std::mutex> lk(m_);
+      open_.store(n, std::memory_order_release);
+    }
+    cv_.notify_all();
+  }
+  void stop() {
+    {
+      std::lock_guard<std::mutex> lk(m_);
+      stop_.store(true, std::memory_order_release);
+    }
+    cv_.notify_all();
+  }
+  bool stopped() const { return stop_.load(std::memory_order_acquire); }
+  // Returns when chunk j is there (true) or the copy is given up.
+  bool wait(size_t j) {
+    if (open_.load(std::memory_order_acquire) > 0) {
+      const auto until = std::chrono::steady_clock::now() + kLook;
+      do {
+        if (open_.load(std::memory_order_acquire) > j) return true;
+        if (stopped()) return false;
+        std::this_thread::yield();
+      } while (std::chrono::steady_clock::now() < until);
+    }
+    std::unique_lock<std::mutex> lk(m_);
+    cv_.wait(lk, [&] { return stopped() || open_.load(std::memory_order_relaxed) > j; });
+    return open_.load(std::memory_order_relaxed) > j;
+  }
+
+ private:
+  static constexpr std::chrono::microseconds kLook{1000};
+  std::mutex m_;
+  std::condition_variable cv_;
+  std::atomic<size_t> open_;
+  std::atomic<bool> stop_{false};
+};
+
 // Threads that run fn until the object goes; none where they cannot start.
 struct Crew {
   std::vector<std::thread> t;
-  std::atomic<bool>& stop;
+  Gate& gate;
   template <class Fn>
-  Crew(std::atomic<bool>& s, int n, Fn fn) : stop(s) {
+  Crew(Gate& g, int n, Fn fn) : gate(g) {
     t.reserve((size_t)n);
     for (int k = 0; k < n; ++k) {
       try {
@@ -124,7 +174,7 @@ struct Crew {
     }
   }
   ~Crew() {
-    stop.store(true, std::memory_order_release);
+    gate.stop();
     for (std::thread& x : t) x.join();
   }
 };
@@ -203,14 +253,12 @@ struct Toucher {
       return;
     }
   }
-  void run(const std::atomic<bool>& stop) {
+  void run(const Gate& gate) {
     for (size_t j; (j = next.fetch_add(1)) < blocks;) {
-      if (!stop.load(std::memory_order_relaxed)) block(j);
+      if (!gate.stopped()) block(j);
       done.fetch_add(1, std::memory_order_release);
     }
-    while (done.load(std::memory_order_acquire) < blocks &&
-           !stop.load(std::memory_order_acquire))
-      pause();
+    while (done.load(std::memory_order_acquire) < blocks && !gate.stopped()) pause();
   }
 };
 
@@ -231,41 +279,33 @@ int drain(const char* dev, const HostPiece* pieces, int count, size_t bytes, con
                                         hipMemcpyDeviceToHost, s);
     return e == hipSuccess ? hipEventRecord(r.event(j), s) : e;
   };
-  std::vector<std::atomic<int>> state(n);  // 1: in its slot, 2: copied out
+  std::vector<std::atomic<bool>> out(n);  // copied out of its slot
   std::atomic<size_t> next{0};
-  std::atomic<bool> stop{false};
+  Gate arrived(0);
   Toucher toucher(pieces, count);
   auto copy = [&](size_t j) {
     move_pieces(pieces, count, j * chunk, end(j), r.slot(j), true);
-    state[j].store(2, std::memory_order_release);
+    out[j].store(true, std::memory_order_release);
   };
   auto work = [&]() {
-    toucher.run(stop);
-    for (;;) {
-      const size_t j = next.fetch_add(1);
-      if (j >= n) return;
-      while (state[j].load(std::memory_order_acquire) == 0) {
-        if (stop.load(std::memory_order_acquire)) return;
-        pause();
-      }
-      copy(j);
-    }
+    toucher.run(arrived);
+    for (size_t j; (j = next.fetch_add(1)) < n && arrived.wait(j);) copy(j);
   };
-  Crew crew(stop, kWorkers, work);
+  Crew crew(arrived, kWorkers, work);
   for (size_t j = 0; j < n && j < kSlots; ++j) LBM_HIP(issue(j));
   for (size_t j = 0; j < n; ++j) {
     LBM_HIP(hipEventSynchronize(r.event(j)));
-    state[j].store(1, std::memory_order_release);
+    arrived.raise(j + 1);
     if (crew.t.empty()) copy(j);
     // the slot takes chunk j + kSlots once its own is out; the crew is
     // several chunks behind at most, so look at the oldest first
     if (j + kSlots < n) {
-      while (state[j].load(std::memory_order_acquire) != 2) pause();
+      while (!out[j].load(std::memory_order_acquire)) pause();
       LBM_HIP(issue(j + kSlots));
     }
   }
   for (size_t j = n > kSlots ? n - kSlots : 0; j < n; ++j)
-    while (state[j].load(std::memory_order_acquire) != 2) pause();
+    while (!out[j].load(std::memory_order_acquire)) pause();
   return LBM_OK;
 }
 
@@ -274,32 +314,24 @@ int feed(char* dev, const HostPiece* pieces, int count, size_t bytes, const Ring
          hipStream_t s) {
   const size_t chunk = chunk_bytes(bytes), n = (bytes + chunk - 1) / chunk;
   auto end = [&](size_t j) { return std::min(bytes, (j + 1) * chunk); };
-  std::vector<std::atomic<int>> full(n);
-  std::atomic<size_t> next{0}, free_below{std::min<size_t>(n, kSlots)};
-  std::atomic<bool> stop{false};
+  std::vector<std::atomic<bool>> full(n);
+  std::atomic<size_t> next{0};
+  Gate free(std::min<size_t>(n, kSlots));
   auto fill = [&](size_t j) {
     move_pieces(pieces, count, j * chunk, end(j), r.slot(j), false);
-    full[j].store(1, std::memory_order_release);
+    full[j].store(true, std::memory_order_release);
   };
   auto work = [&]() {
-    for (;;) {
-      const size_t j = next.fetch_add(1);
-      if (j >= n) return;
-      while (free_below.load(std::memory_order_acquire) <= j) {
-        if (stop.load(std::memory_order_acquire)) return;
-        pause();
-      }
-      fill(j);
-    }
+    for (size_t j; (j = next.fetch_add(1)) < n && free.wait(j);) fill(j);
   };
-  Crew crew(stop, kWorkers, work);
+  Crew crew(free, kWorkers, work);
   for (size_t j = 0; j < n; ++j) {
     if (j >= kSlots) {
       LBM_HIP(hipEventSynchronize(r.event(j)));
-      free_below.store(j + 1, std::memory_order_release);
+      free.raise(j + 1);
     }
     if (crew.t.empty()) fill(j);
-    while (full[j].load(std::memory_order_acquire) == 0) pause();
+    while (!full[j].load(std::memory_order_acquire)) pause();
     LBM_HIP(hipMemcpyAsync(dev + j * chunk, r.slot(j), end(j) - j * chunk, hipMemcpyHostToDevice, s));
     LBM_HIP(hipEventRecord(r.event(j), s));
   }

@@ -153,3 +153,21 @@ def test_memory_of_the_runtime_is_copied_directly(kind):
             assert np.array_equal(c.populations(), f[:27 * n])
     finally:
         (rt.hipHostFree if kind == "pinned" else rt.hipFree)(p)
+
+
+def test_threads_sleep_while_the_gpu_steps():
+    # a result behind queued steps: the copy's threads touch its pages and
+    # sleep until its first chunk is there (they kept six CPUs busy)
+    say("case: CPU time of a read-back behind queued steps")
+    with capi.Context(flat(256 << 20)) as c:
+        c.init_equilibrium()
+        c.step(40)
+        want = c.moments()
+        c.step(2400)
+        t0, p0 = time.perf_counter(), time.process_time()
+        got = c.moments()
+        wall, cpu = time.perf_counter() - t0, time.process_time() - p0
+    say(f"  {cpu:.3f} s of CPU in {wall:.3f} s")
+    assert wall > 0.1  # the steps were still under way
+    assert cpu < 2.5 * wall
+    assert np.array_equal(got[0], want[0])  # rest stays at rest
