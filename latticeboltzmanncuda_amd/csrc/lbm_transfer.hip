@@ -15,9 +15,19 @@
 // fresh array 0.5 against 1.4 ms).
 //
 // Slots (one of 512 KiB for a small copy, a ring of 32 MiB for a large one)
-// are taken from a pool that keeps at most kKept of each; each call has its
-// slots to itself, so calls of several threads and streams do not meet.  The
-// pool is emptied when the last context goes.
+// come from a pool; each call has its slots to itself, so calls of several
+// threads and streams do not meet.  A ring costs 0.1 to 0.6 ms to pin and its
+// first copy 1 to 5 ms more than the following ones, so
+//  - the first is made once 4 small copies or 64 MiB have gone by, before
+//    which the runtime copies;
+//  - at most 8 and 2 of them exist (68 MiB): a call that finds none free
+//    leaves its copy to the runtime;
+//  - when the last context goes, one of each kind stays if a copy asked for it
+//    since the last time, and goes too if none did.
+// So a program that makes a lattice, reads it and destroys it, again and again,
+// finds its slots there.  Its read-back, by the runtime / through slots made
+// anew for each / so: 9 MiB 0.58 / 1.7 / 0.57 ms, 33 MiB 2.0 / 6.4 / 1.0, 256
+// MiB 26 / 25 / 12.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,7 +45,6 @@ namespace lbm {
 namespace {
 
 constexpr int kSlots = 8;
-constexpr size_t kKept = 2;
 // below this the runtime's copy is as fast (64 KiB: 12 us either way)
 constexpr size_t kDirect = 64u << 10;
 // from here on several threads pay for their start (about 0.1 ms)
@@ -58,9 +67,6 @@ struct Slots {
   char* base;
   hipEvent_t ev[kSlots];
 };
-std::mutex g_pool_mutex;
-std::vector<Slots> g_pool;
-int64_t g_contexts = 0;
 
 void free_slots(const Slots& r) {
   for (hipEvent_t e : r.ev)
@@ -68,22 +74,44 @@ void free_slots(const Slots& r) {
   if (r.base) (void)hipHostFree(r.base);
 }
 
-// A ring of slots (with an event each) for one call.
+// The slots of one kind, in use and idle.
+struct Pool {
+  const int most;     // so many at a time
+  const size_t earn;  // copies (small) or bytes (large) until the first is made
+  int made = 0;
+  size_t went = 0;    // copies or bytes so far
+  bool used = false;  // a copy came since the last context went
+  std::vector<Slots> idle;
+};
+constexpr int kMostSmall = 8, kMostLarge = 2;
+std::mutex g_pool_mutex;
+Pool g_small{kMostSmall, 4, 0, 0, false, {}};
+Pool g_large{kMostLarge, 64u << 20, 0, 0, false, {}};
+int64_t g_contexts = 0;
+
+// Slots (with an event each for a large copy) for one call, or none: then
+// the runtime copies.
 struct Ring {
   Slots r{};
   bool ok = false;
-  explicit Ring(bool large) {
+  Ring(bool large, size_t bytes) {
+    Pool& pool = large ? g_large : g_small;
     r.large = large;
     if (hipGetDevice(&r.device) != hipSuccess) return;
     {
       std::lock_guard<std::mutex> lk(g_pool_mutex);
-      for (size_t k = 0; k < g_pool.size(); ++k)
-        if (g_pool[k].device == r.device && g_pool[k].large == large) {
-          r = g_pool[k];
-          g_pool.erase(g_pool.begin() + (std::ptrdiff_t)k);
+      pool.went += large ? bytes : 1;
+      pool.used = true;
+      for (size_t k = 0; k < pool.idle.size(); ++k)
+        if (pool.idle[k].device == r.device) {
+          r = pool.idle[k];
+          pool.idle.erase(pool.idle.begin() + (std::ptrdiff_t)k);
           ok = true;
           return;
         }
+      if (pool.made >= pool.most || pool.went < pool.earn) return;
+      pool.idle.reserve((size_t)pool.most);  // giving back allocates nothing
+      ++pool.made;
     }
     ok = hipHostMalloc((void**)&r.base, large ? kSlots * kLargeSlot : kSmallSlot,
                        hipHostMallocDefault) == hipSuccess;
@@ -91,20 +119,19 @@ struct Ring {
     for (hipEvent_t& e : r.ev)
       if (ok && large) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (!ok) (void)hipGetLastError();
+    std::lock_guard<std::mutex> lk(g_pool_mutex);
+    if (!ok) {
+      --pool.made;
+      pool.went = 0;
+      free_slots(r);
+    }
   }
   Ring(const Ring&) = delete;
   Ring& operator=(const Ring&) = delete;
   ~Ring() {
-    {
-      std::lock_guard<std::mutex> lk(g_pool_mutex);
-      size_t kept = 0;
-      for (const Slots& other : g_pool) kept += other.large == r.large;
-      if (ok && g_contexts > 0 && kept < kKept) {
-        g_pool.push_back(r);
-        return;
-      }
-    }
-    free_slots(r);
+    if (!ok) return;
+    std::lock_guard<std::mutex> lk(g_pool_mutex);
+    (r.large ? g_large : g_small).idle.push_back(r);
   }
   char* slot(size_t j) const { return r.base + (j % kSlots) * kLargeSlot; }
   hipEvent_t event(size_t j) const { return r.ev[j % kSlots]; }
@@ -345,7 +372,7 @@ int transfer(char* dev, const HostPiece* pieces, int count, bool out, hipStream_
   const bool large = bytes >= (out ? kThreaded : kFeed);
   const bool small = out && bytes >= kDirect && bytes <= kSmallSlot;
   if ((!large && !small) || !ordinary(pieces, count)) return plain(dev, pieces, count, out, s);
-  Ring ring(large);
+  Ring ring(large, bytes);
   if (!ring.ok) return plain(dev, pieces, count, out, s);
   const int rc = out ? drain(dev, pieces, count, bytes, ring, s)
                      : feed(dev, pieces, count, bytes, ring, s);
@@ -370,13 +397,24 @@ int copy_to_host_plain(const void* dev, const HostPiece* pieces, int count, hipS
 }
 
 void transfer_context(int delta) {
-  std::vector<Slots> drop;
+  Slots drop[kMostSmall + kMostLarge];
+  size_t count = 0;
   {
     std::lock_guard<std::mutex> lk(g_pool_mutex);
     g_contexts += delta;
-    if (g_contexts == 0) drop.swap(g_pool);
+    if (g_contexts > 0 || delta > 0) return;
+    for (Pool* pool : {&g_small, &g_large}) {
+      const size_t keep = pool->used ? 1 : 0;
+      while (pool->idle.size() > keep) {
+        drop[count++] = pool->idle.back();
+        pool->idle.pop_back();
+        --pool->made;
+      }
+      if (!pool->used) pool->went = 0;
+      pool->used = false;
+    }
   }
-  for (const Slots& r : drop) free_slots(r);
+  for (size_t k = 0; k < count; ++k) free_slots(drop[k]);
 }
 
 }  // namespace lbm

@@ -171,3 +171,30 @@ def test_threads_sleep_while_the_gpu_steps():
     assert wall > 0.1  # the steps were still under way
     assert cpu < 2.5 * wall
     assert np.array_equal(got[0], want[0])  # rest stays at rest
+
+
+@pytest.mark.parametrize("nbytes", [200 << 10, 9 << 20])
+def test_more_threads_than_slots(nbytes):
+    say(f"case: 12 threads read {nbytes >> 10} KiB each")
+    cs = [capi.Context(flat(nbytes)) for _ in range(12)]
+    want, errors = [], []
+    for k, c in enumerate(cs):
+        c.init_equilibrium(np.full(c.n, 1.0 + 0.001 * k))
+        want.append(np.float32(c.moments()[0][0]))
+
+    def work(k):
+        try:
+            for _ in range(6):
+                rho, u = cs[k].moments()
+                assert (rho == want[k]).all() and (u == 0).all()
+        except BaseException as e:  # noqa: BLE001 (reported below)
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(12)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for c in cs:
+        c.close()
+    assert not errors, errors
