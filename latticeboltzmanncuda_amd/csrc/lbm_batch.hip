@@ -230,15 +230,16 @@ int sweep_grid(const lbm_batch* b) {
   return (int)((wg + 255) / 256 * 256);
 }
 
-// n steps of class k on stream s.
-int launch_class(lbm_batch* b, int k, int n, hipStream_t st) {
+// n steps of class k on stream s; single: one step a launch, whatever the
+// class takes otherwise.
+int launch_class(lbm_batch* b, int k, int n, hipStream_t st, bool single = false) {
   const int storage = device_storage(LBM_MODE_STANDARD, b->storage);
   const int grid = class_grid(b, k);
   if (grid == 0) return LBM_OK;
   // launches of one step each, or for the D2Q9 lattices passes of up to
   // four; as many passes, odd or even, as there are steps, so that every
   // member's current buffer is the same one
-  const int passes = k == 0 && b->nunits ? sweep_passes(n) : n;
+  const int passes = k == 0 && b->nunits && !single ? sweep_passes(n) : n;
   for (int s = 0, left = n; s < passes; ++s) {
     const int steps = (left + (passes - s) - 1) / (passes - s);
     const int rc =
@@ -297,8 +298,9 @@ int each_class(lbm_batch* b, bool aside, Go&& go) {
 // Below this many steps a second stream's events cost more than it gives (a
 // chunk of 10 steps 15.5 against 15.9 us per step, of 20 12.8 / 15.6).
 constexpr int kSideSteps = 10;
-int launch_steps(lbm_batch* b, int n) {
-  return each_class(b, n >= kSideSteps, [&](int k, hipStream_t s) { return launch_class(b, k, n, s); });
+int launch_steps(lbm_batch* b, int n, bool single = false) {
+  return each_class(b, n >= kSideSteps,
+                    [&](int k, hipStream_t s) { return launch_class(b, k, n, s, single); });
 }
 
 void advance_members(lbm_batch* b, int n) {
@@ -665,6 +667,11 @@ int lbm_batch_autotune(lbm_batch* b, int steps, int use_cache, int* block_out,
     if (grid_out) *grid_out = b->grid;
     return LBM_OK;
   }
+  // Timed by single steps: the shape is that of the tile kernels, which take
+  // the steps that a sweep leaves over, and the cache hands it to batches of
+  // this size that take all their steps so.  (Timed by sweeps, which do not
+  // use it, every shape took the same: 256 lattices of 32 to 512 a side got
+  // one with which two single steps took 242 us instead of 164.)
   float best = 0.0f;
   int best_block = b->block, best_grid = b->grid;
   bool have = false;
@@ -677,9 +684,9 @@ int lbm_batch_autotune(lbm_batch* b, int steps, int use_cache, int* block_out,
       if (b->grid == 0 && block == 64) continue;
       int rc = sync_tables(b);
       if (rc) return rc;
-      if ((rc = launch_steps(b, 2))) return rc;  // warm-up (even)
+      if ((rc = launch_steps(b, 2, true))) return rc;  // warm-up (even)
       LBM_HIP(hipEventRecord(b->ev0, b->stream));
-      if ((rc = launch_steps(b, steps))) return rc;
+      if ((rc = launch_steps(b, steps, true))) return rc;
       launched += steps + 2;
       LBM_HIP(hipEventRecord(b->ev1, b->stream));
       LBM_HIP(hipEventSynchronize(b->ev1));

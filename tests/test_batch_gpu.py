@@ -2,6 +2,7 @@
 launches and hipGraph chunks) give the same populations as each lattice
 stepped alone; admission honours the HBM budget; residuals are right."""
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -193,3 +194,37 @@ def test_classes_side_by_side_equal_alone(calls):
         assert np.array_equal(late.populations(), run_alone(*specs[5], 40))
         assert np.array_equal(members[6].populations(),
                               run_alone(*specs[6], done + 40))
+
+
+@pytest.mark.parametrize("storage,side", [(capi.STORE_F32, 1400),
+                                          (capi.STORE_F64, 1400),
+                                          (capi.STORE_F16, 2500)])
+def test_autotuner_times_the_kernel_whose_shape_it_chooses(storage, side):
+    # large D2Q9 batches take several steps a launch in a kernel of one shape;
+    # the tuner's shape is for the other one, so its 19 candidates take at
+    # least as long as single steps
+    say(f"case: autotuner on a batch of sweeps, storage {storage}")
+    steps = 60
+    cfg = capi.make_config(side, side, 1, lattice=9, storage=storage, tau=0.7,
+                           periodic=(1, 0, 0), force=(1e-6, 0, 0))
+    with capi.Batch(storage) as b:
+        m = b.add(cfg)
+        b.step(10)
+        b.synchronize()
+        t0 = time.perf_counter()
+        b.autotune(steps, use_cache=False)
+        tuning = time.perf_counter() - t0
+        single = 1e9
+        for _ in range(3):
+            t0 = time.perf_counter()
+            for _ in range(steps // 2):
+                b.step(2)
+            b.synchronize()
+            single = min(single, (time.perf_counter() - t0) / steps)
+        b.step(30)
+        b.synchronize()
+        got = m.populations()
+    say(f"  tuning {tuning * 1e3:.1f} ms, a single step {single * 1e6:.1f} us")
+    assert tuning > 0.85 * 19 * steps * single
+    total = 10 + 19 * (steps + 2) + 3 * steps + 30
+    assert np.array_equal(got, run_alone(cfg, None, total))
