@@ -120,11 +120,11 @@ struct lbm_batch {
   int tables_block = 0;  // block size the tile table was built for
   bool nt = false;       // non-temporal stores: members exceed the Infinity Cache
 
-  // captured chunk, by class
+  // captured chunk, by class, or (whole) all classes in the first one's graph
   hipGraph_t graph[lbm::kBatchClasses] = {};
   hipGraphExec_t graph_exec[lbm::kBatchClasses] = {};
   int graph_chunk = 0, graph_block = 0;  // 0 steps: none captured
-  bool graph_nt = false;
+  bool graph_nt = false, graph_whole = false;
   const void* graph_lats = nullptr;    // descriptor table the graph reads
   const void* graph_ntiles = nullptr;  // tile counts the graph reads
   // per class: tile table and grid the captured launches use (null / 0 for

@@ -342,14 +342,20 @@ void advance_members(lbm_batch* b, int n) {
 
 // One graph per class: graphs without branches, which need no streams of
 // their own (a graph with a branch per class took 4 ms more to instantiate
-// and destroy).
-int capture_chunk(lbm_batch* b, int chunk) {
+// and destroy).  whole: all classes in one graph, that of the first, for calls
+// that step on one stream and for chunks of two steps (six lattices of 64 to
+// 200 a side, D2Q9 and D3Q19, a graph per class against one: a call of two
+// steps 34.6 / 29.7 us, of ten in chunks of two 136-213 / 149, of 16 in chunks
+// of eight 178 / 199).
+int capture_chunk(lbm_batch* b, int chunk, bool whole) {
   drop_graph(b);
   for (int k = 0; k < kBatchClasses; ++k) {
     if (class_grid(b, k) == 0) continue;
     hipError_t e = hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(e, "hipStreamBeginCapture");
-    const int rc = launch_class(b, k, chunk, b->stream);
+    int rc = LBM_OK;
+    for (int j = k; j < (whole ? kBatchClasses : k + 1) && !rc; ++j)
+      rc = launch_class(b, j, chunk, b->stream);
     e = hipStreamEndCapture(b->stream, &b->graph[k]);
     if (rc) {
       drop_graph(b);
@@ -360,8 +366,10 @@ int capture_chunk(lbm_batch* b, int chunk) {
       drop_graph(b);
       return hip_fail(e, "capture of a chunk");
     }
+    if (whole) break;
   }
   b->graph_chunk = chunk;
+  b->graph_whole = whole;
   b->graph_block = b->block;
   b->graph_nt = b->nt;
   b->graph_lats = b->d_lats;
@@ -394,9 +402,11 @@ bool graph_current(const lbm_batch* b, int chunk) {
   return true;
 }
 
-int ensure_graph(lbm_batch* b, int chunk) {
+// steps: those of the call that captures, which says how its classes go; later
+// calls take the graphs that are there.
+int ensure_graph(lbm_batch* b, int chunk, int steps) {
   if (graph_current(b, chunk)) return LBM_OK;
-  return capture_chunk(b, chunk);
+  return capture_chunk(b, chunk, steps < kSideSteps || chunk < 4);
 }
 
 // Launch-shape cache of the autotuner: (storage, lattice-mix bits, log2
@@ -646,9 +656,11 @@ int lbm_batch_step_graph(lbm_batch* b, int n, int chunk) {
   if (rc || n == 0 || b->ntiles == 0) return rc;
   const int full = n / chunk;
   if (full > 0) {
-    if ((rc = ensure_graph(b, chunk))) return rc;
-    rc = each_class(b, full * chunk >= kSideSteps, [&](int k, hipStream_t s) -> int {
-      for (int c = 0; c < full; ++c) LBM_HIP(hipGraphLaunch(b->graph_exec[k], s));
+    if ((rc = ensure_graph(b, chunk, full * chunk))) return rc;
+    rc = each_class(b, !b->graph_whole && full * chunk >= kSideSteps, [&](int k, hipStream_t s) -> int {
+      // (a class without a graph has its steps in the first one's)
+      for (int c = 0; c < full && b->graph_exec[k]; ++c)
+        LBM_HIP(hipGraphLaunch(b->graph_exec[k], s));
       return LBM_OK;
     });
     if (rc) return rc;
@@ -672,7 +684,7 @@ int lbm_batch_time_steps(lbm_batch* b, int n, int chunk, float* ms) {
     return fail(LBM_ERR_INVALID, "chunk must be an even step count >= 2");
   int rc = sync_tables(b);
   if (rc) return rc;
-  if (chunk > 0 && b->ntiles > 0 && (rc = ensure_graph(b, chunk))) return rc;
+  if (chunk > 0 && b->ntiles > 0 && (rc = ensure_graph(b, chunk, n / chunk * chunk))) return rc;
   LBM_HIP(hipEventRecord(b->ev0, b->stream));
   rc = chunk > 0 ? api::lbm_batch_step_graph(b, n, chunk) : api::lbm_batch_step(b, n);
   if (rc) return rc;

@@ -279,3 +279,44 @@ def test_many_members_step_and_change(tmp_path):
         c.load(path)
         c.step(17)
         assert np.array_equal(got[4], c.populations())
+
+
+def test_short_chunks_of_several_types_cost_no_more_than_their_launches():
+    # chunks of two steps hold all lattice types in one graph: with one graph
+    # per type and chunk they took up to 1.4 times as long
+    say("case: short chunks of two lattice types")
+    specs = [(capi.make_config(90, 80 + k, 1, lattice=9, tau=0.7, lid_face=3,
+                               lid_u=(0.05, 0, 0)), None) for k in range(6)]
+    specs += [(capi.make_config(20, 22, 20 + k, lattice=19, tau=0.7,
+                                periodic=(1, 0, 0), force=(1e-5, 0, 0)), None)
+              for k in range(6)]
+
+    def members(select):
+        b = capi.Batch(capi.STORE_F32)
+        ms = [b.add(*s) for s in specs if select(s[0].lattice)]
+        b.step(20, 2)
+        b.synchronize()
+        return b, ms
+
+    def took(b):
+        best = 1e9
+        for _ in range(5):
+            t0 = time.perf_counter()
+            for _ in range(20):
+                b.step(20, 2)
+            b.synchronize()
+            best = min(best, (time.perf_counter() - t0) / 20)
+        return best
+
+    both, ms = members(lambda q: True)
+    flat, _ = members(lambda q: q == 9)
+    deep, _ = members(lambda q: q == 19)
+    t = [took(b) * 1e6 for b in (both, flat, deep)]
+    say(f"  20 steps by twos: both {t[0]:.0f} us, D2Q9 {t[1]:.0f}, D3Q19 "
+        f"{t[2]:.0f}")
+    assert t[0] < 0.92 * (t[1] + t[2])
+    got = [m.populations() for m in ms]
+    for b in (both, flat, deep):
+        b.close()
+    for (cfg, solid), g in list(zip(specs, got))[::5]:
+        assert np.array_equal(g, run_alone(cfg, solid, 20 + 5 * 20 * 20))
