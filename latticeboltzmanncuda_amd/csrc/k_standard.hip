@@ -619,9 +619,9 @@ bool single_steps() {
 
 int std_box_steps(int q, int storage, const Grid& g) {
   if (q != 9 || single_steps() ||
-      box_wide_count(g) * kBoxWideNodes > box_max_nodes(storage))
+      box_wide_count(g) * kBoxWideNodes > box_max_nodes(storage) || !box_fits(g))
     return 0;
-  return g.n <= box_small_nodes(storage) ? 8 : 4;
+  return g.n <= box_small_nodes(storage) && box_eights_fit(g) ? 8 : 4;
 }
 
 int launch_std_box(int k, int storage, const Grid& g, const void* A, void* B,
@@ -641,7 +641,7 @@ int launch_std_box(int k, int storage, const Grid& g, const void* A, void* B,
 }
 
 bool std_sweeps(int q, int storage, const Grid& g) {
-  if (q != 9 || single_steps()) return false;
+  if (q != 9 || single_steps() || !sweep_fits(g, storage, g.n)) return false;
   // 16-bit lattices that fit the Infinity Cache are as fast one step at a
   // time (2900 x 1700: 24.2-30.5 against 24.7-28.9 us), larger ones are not
   return storage_bytes(storage) == 2 ? streams(q, storage, g) : g.n >= kSweepMinNodes;

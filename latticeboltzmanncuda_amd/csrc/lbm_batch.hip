@@ -77,14 +77,19 @@ bool tables_stale(const lbm_batch* b) {
   return false;
 }
 
-// Whether a batch's D2Q9 members (`nodes` of them all) are stepped by
+// Whether a batch's D2Q9 members are stepped by
 // sweeps: where they fill the GPU with wavefronts that walk a few dozen rows
 // each.  Measured per step, tiles against sweeps: FP32 0.36 M nodes 5.9 / 6.7
 // us, 0.96 M 13.6 / 9.6, 6.7 M 81.8 / 43.4; FP64 0.96 M 22.5 / 12.9, 6.7 M
 // 161 / 76; FP16, whose tiles move half the bytes for the same
-// instructions, 3.5 M 24.2 / 25.0, 6.7 M 55.0 / 45.5.
-bool sweep_batch(int storage, uint64_t nodes) {
-  return nodes >= (storage_bytes(storage) == 2 ? 5000000u : 600000u);
+// instructions, 3.5 M 24.2 / 25.0, 6.7 M 55.0 / 45.5.  Members whose rows do
+// not fit a sweep (sweep_fits) may hold an eighth of the nodes.
+bool sweep_batch(int storage, const std::vector<const lbm_ctx*>& flat) {
+  uint64_t nodes = 0, unfit = 0;
+  for (const lbm_ctx* c : flat) nodes += c->grid.n;
+  for (const lbm_ctx* c : flat)
+    if (!sweep_fits(c->grid, storage, nodes)) unfit += c->grid.n;
+  return nodes >= (storage_bytes(storage) == 2 ? 5000000u : 600000u) && unfit * 8 <= nodes;
 }
 
 // Counters on the device: tiles of each class, sweep units.
@@ -127,13 +132,9 @@ int sync_tables(lbm_batch* b) {
   uint64_t pop_bytes = 0;
   // the D2Q9 members' sweep
   std::vector<const lbm_ctx*> flat;
-  uint64_t flat_nodes = 0;
   for (const lbm_ctx* c : b->slots)
-    if (c && c->q == 9) {
-      flat.push_back(c);
-      flat_nodes += c->grid.n;
-    }
-  const bool sweep = sweep_batch(b->storage, flat_nodes);
+    if (c && c->q == 9) flat.push_back(c);
+  const bool sweep = sweep_batch(b->storage, flat);
   const uint32_t chunk_rows =
       sweep ? sweep_chunk_rows(flat.size(), [&](size_t i) -> const Grid& { return flat[i]->grid; },
                                b->storage)
@@ -268,17 +269,20 @@ int launch_class(lbm_batch* b, int k, int n, hipStream_t st, bool single = false
   // launches of one step each, or for the D2Q9 lattices passes of up to
   // four; as many passes, odd or even, as there are steps, so that every
   // member's current buffer is the same one
-  const int passes = k == 0 && b->nunits && !single ? sweep_passes(n) : n;
-  for (int s = 0, left = n; s < passes; ++s) {
-    const int steps = (left + (passes - s) - 1) / (passes - s);
-    const int rc =
-        steps > 1 ? launch_batch_sweep(storage, steps, sweep_grid(b), b->d_lats, b->d_units,
-                                       b->d_ntiles + kBatchClasses, s & 1, st)
-                  : launch_batch_step(storage, k, b->nt, b->block, grid, b->d_lats, b->d_tiles[k],
-                                      b->d_ntiles + k, s & 1, st);
-    if (rc) return rc;
-    left -= steps;
+  int launches[5] = {0, n, 0, 0, 0};
+  if (k == 0 && b->nunits && !single) {
+    launches[1] = 0;
+    split_steps(n, sweep_costs(storage), launches);
   }
+  for (int steps = 4, pass = 0; steps > 0; --steps)
+    for (int s = 0; s < launches[steps]; ++s, ++pass) {
+      const int rc =
+          steps > 1 ? launch_batch_sweep(storage, steps, sweep_grid(b), b->d_lats, b->d_units,
+                                         b->d_ntiles + kBatchClasses, pass & 1, st)
+                    : launch_batch_step(storage, k, b->nt, b->block, grid, b->d_lats,
+                                        b->d_tiles[k], b->d_ntiles + k, pass & 1, st);
+      if (rc) return rc;
+    }
   return LBM_OK;
 }
 

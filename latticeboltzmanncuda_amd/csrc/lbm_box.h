@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "lbm_step_node.h"
+#include "lbm_sweep.h"
 
 namespace lbm {
 
@@ -71,6 +72,48 @@ inline uint64_t box_wide_count(const Grid& g) {
   return (uint64_t)((g.nx + 15) / 16) * ((g.ny + 15) / 16);
 }
 constexpr uint32_t kBoxWideNodes = 16 * 16;
+
+// Microseconds of a launch of k steps, k of 1 (one step of the lattice by
+// itself) to 4 (BoxWide), fitted to what lattices of 64^2 to 800^2 and thin
+// ones of 20000 x 8 to 60 x 6000 took: a launch of boxes is its start and
+// load latency and so much a box, little less where part of it lies outside
+// the lattice.  So short calls and thin lattices go by single steps where
+// these are faster (FP16 520 x 990 by twos 7.7-8.3 us a step, by threes
+// 5.9-6.9, by fours 4.8-5.7, singly 4.8-6.0; FP32 20000 x 20 by twos 7.2, by
+// fours 5.1, singly 5.9).
+inline StepCosts box_costs(int storage, const Grid& g) {
+  const double n = g.n, whole = (double)(box_wide_count(g) * kBoxWideNodes);
+  const double boxes = (0.6 * whole + 0.4 * n) / kBoxWideNodes;
+  auto most = [](double a, double b) { return a > b ? a : b; };
+  switch (storage_bytes(storage)) {
+    case 2:
+      // (two and three with a margin: where single steps are bound by the host,
+      // they take 2.7 to 3.6 us, as the host's clock is)
+      return {{0.0, most(3.15, 1.2 + 8.5e-6 * n), 1.2 * (5.5 + 0.0050 * boxes),
+               1.1 * (5.4 + 0.0064 * boxes), 5.8 + 0.0066 * boxes}};
+    case 8:
+      return {{0.0, most(3.7, 2.0 + 24e-6 * n), 5.2 + 0.0098 * boxes, 6.5 + 0.0115 * boxes,
+               7.5 + 0.0127 * boxes}};
+    default:
+      return {{0.0, most(3.3, 2.6 + 10e-6 * n), 4.6 + 0.0056 * boxes, 5.8 + 0.0067 * boxes,
+               6.5 + 0.0072 * boxes}};
+  }
+}
+
+// Thin lattices fill little of their boxes, whose cells beyond a wall idle:
+// where that leaves more than two boxes a CU, single steps are faster below a
+// fifth (per step singly / by boxes, FP32 40000 x 1 3.2 / 7.4 us, 2 x 50000
+// 3.4 / 3.9, 5000 x 4 3.3 / 1.3) and fours than eights below six tenths (FP64
+// 10000 x 8 singly 4.5, by eights 4.9).
+constexpr uint64_t kBoxesAny = 512;
+inline bool box_fits(const Grid& g) {
+  const uint64_t boxes = box_wide_count(g);
+  return boxes <= kBoxesAny || boxes * kBoxWideNodes <= 5ull * g.n;
+}
+inline bool box_eights_fit(const Grid& g) {
+  const uint64_t boxes = box_wide_count(g);
+  return boxes <= kBoxesAny || 6 * boxes * kBoxWideNodes <= 10ull * g.n;
+}
 
 template <class X, class T>
 struct BoxShared {

@@ -21,6 +21,7 @@
 #include "lbm_lattice.h"
 #include "lbm_layout.h"
 #include "lbm_store.h"
+#include "lbm_box.h"
 #include "lbm_march.h"
 #include "lbm_sweep.h"
 
@@ -330,17 +331,12 @@ StepPlan plan_steps(int q, int storage, const Grid& g, int n) {
     return p;
   }
   const int box = std_box_steps(q, storage, g);
-  int rest = n;  // taken as evenly as can be
   if (box || std_sweeps(q, storage, g)) {
     p.kernel = box ? LBM_STEP_BOX : LBM_STEP_SWEEP;
     // boxes of 8 steps come in pairs
     if (box == 8) p.launches[8] = n / 16 * 2;
-    rest -= 8 * p.launches[8];
-    for (int passes = sweep_passes(rest); passes > 0; --passes) {
-      const int k = (rest + passes - 1) / passes;
-      ++p.launches[k];
-      rest -= k;
-    }
+    split_steps(n - 8 * p.launches[8], box ? box_costs(storage, g) : sweep_costs(storage),
+                p.launches);
     if (!box)
       p.sweep = sweep_plan(g, sweep_chunk_rows(1, [&](size_t) -> const Grid& { return g; }, storage));
   } else if (n >= 4 && std_marches(q, storage, g, &p.march)) {

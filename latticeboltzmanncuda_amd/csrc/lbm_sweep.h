@@ -140,12 +140,63 @@ uint32_t sweep_chunk_rows(size_t count, GridOf&& grid, int storage) {
 // after another.
 constexpr uint32_t kSweepMinNodes = 200000;
 
-// Passes for n steps, as odd or even as n and as even in length as they can
-// be: n / passes steps each, the first n % passes one more.  At most 4 steps
-// a pass (a fifth stage's registers leave too few wavefronts).
-inline int sweep_passes(int n) {
-  const int p = (n + 3) / 4;
-  return ((p ^ n) & 1) ? p + 1 : p;
+// Whether a lattice's rows are long enough, and enough of them, for a sweep;
+// nodes: of all that are swept together.  Several chunks of short rows share
+// a wavefront, whose loads and stores then scatter: per step against one at a
+// time, FP32 rows of 1 / 2 / 4 / 8 / 16 nodes 6 M nodes 5.6 / 3.2 / 1.4 / 0.79
+// / 0.51, 1 M nodes 6.2 / 3.0 / 1.4 / 1.4 / 0.83; FP64 6 M 3.0 / 1.5 / 0.82 /
+// 0.49 / 0.38, 1 M 3.8 / 1.7 / 1.4 / 1.4 / 0.79; FP16 9 M rows of 8 / 16 / 24
+// 1.4 / 0.9-1.1 / 0.85.  A chunk of few rows is mostly rim: a single row FP32
+// 6 M 1.35, two 0.74; FP16 9 M 2 / 4 / 8 rows 1.4-1.6 / 0.97-1.1 / 0.8.
+inline bool sweep_fits(const Grid& g, int storage, uint64_t nodes) {
+  const size_t bytes = storage_bytes(storage);
+  if (bytes == 2) return g.nx >= 8 && g.ny >= 24;
+  const uint32_t row = nodes >= 4000000 && bytes == 8 ? 4 : nodes >= 2000000 ? 8 : 16;
+  return g.nx >= 2 && g.ny >= row;
+}
+
+// What a launch of k steps costs ([k], k of 1 to 4), in any unit.
+struct StepCosts {
+  double of[5];
+};
+// Sweeps, in single steps (medians over 0.2 to 17 M nodes): two steps a pass
+// save little, with 16 bits nothing, so a call of 4 goes by 3 and 1 (4096^2
+// FP16 channel 449 -> 390 us; by twos it was slower than by ones).
+inline StepCosts sweep_costs(int storage) {
+  switch (storage_bytes(storage)) {
+    case 2: return {{0.0, 1.0, 2.05, 2.25, 2.9}};
+    case 8: return {{0.0, 1.0, 1.45, 1.5, 1.8}};
+    default: return {{0.0, 1.0, 1.6, 1.75, 2.2}};
+  }
+}
+
+// Splits n steps into launches of 1 to 4 (launches[k]: how many of k steps) at
+// the least cost.  As many launches, odd or even, as there are steps, so that
+// the current buffer is the one after single steps: those of 2 and 4 are even
+// in number together.
+inline void split_steps(int n, const StepCosts& c, int* launches) {
+  const int most = c.of[4] < 4 * c.of[1] ? 4 : 1;
+  if (n > 24) {  // the bulk of a long call
+    const int eights = (n - 16) / 8;
+    launches[most] += 8 / most * eights;
+    n -= 8 * eights;
+  }
+  double best = 0.0;
+  int take[5] = {0, -1, 0, 0, 0};
+  for (int f = n / 4; f >= 0; --f)
+    for (int t = (n - 4 * f) / 3; t >= 0; --t)
+      for (int w = (n - 4 * f - 3 * t) / 2; w >= 0; --w) {
+        if ((f + w) & 1) continue;
+        const int o = n - 4 * f - 3 * t - 2 * w;
+        const double cost = f * c.of[4] + t * c.of[3] + w * c.of[2] + o * c.of[1];
+        if (take[1] >= 0 && cost >= best) continue;
+        best = cost;
+        take[1] = o;
+        take[2] = w;
+        take[3] = t;
+        take[4] = f;
+      }
+  for (int k = 1; k <= 4; ++k) launches[k] += take[k];
 }
 
 // v of the next lane (y + 1) / of the previous one (y - 1); 0 past the ends

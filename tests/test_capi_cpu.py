@@ -208,3 +208,42 @@ def test_early_loads_only_where_they_are_faster():
         kernel, by = capi.step_route(
             capi.make_config(*dims, lattice=q, storage=storage, tau=0.7), 100)
         assert (kernel, by) == (want, {1: 100}), (q, storage, dims)
+
+
+def test_several_steps_a_launch_only_where_they_are_faster():
+    # shapes and calls that were slower by several steps a launch than singly
+    F32, F64, F16, BF16 = (capi.STORE_F32, capi.STORE_F64, capi.STORE_F16,
+                           capi.STORE_BF16)
+    box, sweep = capi.STEP_BOX, capi.STEP_SWEEP
+
+    def route(dims, storage, n):
+        return capi.step_route(capi.make_config(
+            *dims, 1, lattice=9, storage=storage, tau=0.7), n)
+
+    # rows too short for a sweep, or too few of them, and boxes mostly empty
+    for dims, storage in (((6000000, 1), F32), ((3000000, 2), F32),
+                          ((1, 3000000), F32), ((1500000, 4), F32),
+                          ((125000, 8), F64), ((250000, 4), F64),
+                          ((3000000, 2), F64), ((562500, 16), F16),
+                          ((4, 2250000), BF16), ((20000, 20), F16),
+                          ((40000, 1), F32), ((2, 50000), BF16)):
+        for n in (2, 3, 4, 7, 16, 1000):
+            kernel, by = route(dims, storage, n)
+            assert by == {1: n} and kernel not in (box, sweep), (dims, n)
+    # long rows, and short ones of many nodes
+    for dims, storage in (((750000, 8), F32), ((1500000, 4), F64),
+                          ((62500, 16), F32), ((375000, 24), F16),
+                          ((8, 1125000), F16), ((2, 3000000), F32)):
+        kernel, by = route(dims, storage, 1000)
+        assert kernel == sweep and by == {4: 250}, (dims, by)
+    # calls of a few steps: by 3 and 1, not by twos; with 16 bits singly
+    for dims, storage in (((330, 330), F32), ((900, 900), F64),
+                          ((4096, 4096), F16), ((4096, 4096), F32),
+                          ((300, 300), BF16)):
+        assert route(dims, storage, 4)[1] == {3: 1, 1: 1}, dims
+        assert route(dims, storage, 5)[1] == {3: 1, 1: 2}, dims
+        assert route(dims, storage, 2)[1] == {1: 2}, dims
+    for dims in ((600, 600), (520, 990), (800, 800)):
+        for n in (2, 3, 4, 5, 6, 7):
+            assert route(dims, F16, n)[1] == {1: n}
+        assert route(dims, F16, 8) == (box, {4: 2})
