@@ -246,6 +246,16 @@ bool mesh_closes(const float* vertices, const int32_t* faces, int32_t nf) {
   return open == 0;
 }
 
+// Whether no node of the lattice lies in the box [lo, hi].
+bool box_is_empty(const Grid& g, float spacing, const float3& lo, const float3& hi) {
+  if (!(spacing > 0.0f) || !std::isfinite(spacing)) return false;
+  auto along = [&](float a, float b, uint32_t n) {  // (with room for rounding)
+    return std::max(0.0, std::ceil((double)a / spacing - 1e-3)) <=
+           std::min((double)n - 1.0, std::floor((double)b / spacing + 1e-3));
+  };
+  return !(along(lo.x, hi.x, g.nx) && along(lo.y, hi.y, g.ny) && along(lo.z, hi.z, g.nz));
+}
+
 // ---------------------------------------------------------------------
 // lbm_build_reflections: the reflection tables of preProcessModel
 // (reference Lattice.cpp:323-426, 450-477) on the GPU, one wavefront per
@@ -613,7 +623,10 @@ int lbm_voxelize_mesh(lbm_ctx* c, const float* vertices, int32_t nv,
   uint8_t* dout = mem.at<uint8_t>(o_in);
   LBM_HIP(hipMemcpyAsync(dv, vertices, 12 * (size_t)nv, hipMemcpyHostToDevice, c->stream));
   LBM_HIP(hipMemcpyAsync(df, faces, 12 * (size_t)nf, hipMemcpyHostToDevice, c->stream));
-  const bool closes = mesh_closes(vertices, faces, nf);
+  // where no node lies in the mesh's box no face is tested, and whether the
+  // mesh closes need not be known (14,160 faces: 85 us, with the look at their
+  // edges 199)
+  const bool closes = !box_is_empty(g, spacing, lo, hi) && mesh_closes(vertices, faces, nf);
   if (closes) {
     unsigned long long* dn = mem.at<unsigned long long>(o_n);
     Box* db = mem.at<Box>(o_b);
