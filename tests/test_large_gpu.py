@@ -69,3 +69,29 @@ def test_streaming_store_d2q9_f16_cavity():
     du = np.abs(ug[0] - uo[0]).max() / np.abs(uo[0]).max()
     say(f"  u rel diff {du:.2e}")
     assert du < 2e-3
+
+
+@pytest.mark.parametrize("dims", [(2800, 2800), (2801, 2798)])
+def test_group_step_of_a_large_lattice_equals_one_node_steps(dims):
+    # one step a call: four (or two) nodes per thread with non-temporal
+    # stores, which calls of several steps no longer take at this size
+    say(f"case: group step {dims}")
+    rng = np.random.default_rng(8)
+    solid = (rng.random(dims[0] * dims[1]) < 0.05).astype(np.uint8)
+    cfg = capi.make_config(*dims, 1, lattice=9, storage=capi.STORE_F16,
+                           tau=0.7, lid_face=3, lid_u=(0.1, 0, 0))
+    assert capi.step_route(cfg, 1) == (capi.STEP_GROUP, {1: 1})
+    got = []
+    for env in (None, "0"):
+        if env is not None:
+            os.environ["LBM_GROUP_STEP"] = env
+        try:
+            with capi.Context(cfg) as c:
+                c.upload_solid(solid)
+                c.init_equilibrium()
+                for _ in range(6):
+                    c.step(1)
+                got.append(c.populations())
+        finally:
+            os.environ.pop("LBM_GROUP_STEP", None)
+    assert np.array_equal(*got)

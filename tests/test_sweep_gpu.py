@@ -111,3 +111,37 @@ def test_large_lattice_sweep_equals_single_steps(dims, per, storage):
         finally:
             os.environ.pop("LBM_GROUP_STEP", None)
     assert np.array_equal(*got)
+
+
+# above the sizes that are stepped in boxes, and rows of 8 to 16 nodes
+@pytest.mark.parametrize("dims,per,storage", [
+    ((1201, 701), (0, 0, 0), F32),     # strips with a remainder
+    ((17001, 50), (0, 1, 0), F32),     # one strip with its halo, periodic
+    ((4001, 233), (1, 0, 0), F32),
+    ((62501, 16), (1, 0, 0), F32),     # several chunks a wavefront
+    ((2, 400000), (1, 1, 0), F32),     # two rows
+    ((901, 777), (1, 1, 0), F64),
+    ((250001, 8), (0, 0, 0), F64),
+    ((23, 30011), (0, 0, 0), F64)])
+def test_sweep_above_the_boxes_equals_single_steps(dims, per, storage):
+    say(f"case: sweep above the boxes {dims} periodic {per} storage {storage}")
+    n = dims[0] * dims[1]
+    rng = np.random.default_rng(6)
+    solid = (rng.random(n) < 0.1).astype(np.uint8)
+    kw = dict(lid_face=3, lid_u=(0.05, 0, 0)) if not per[1] else {}
+    cfg = capi.make_config(*dims, 1, lattice=capi.D2Q9, storage=storage,
+                           tau=0.8, periodic=per, force=(1e-5, 0, 0), **kw)
+    assert capi.step_route(cfg, 8) == (capi.STEP_SWEEP, {4: 2})
+    rho = 1.0 + 0.01 * rng.random(n)
+    u = 0.02 * (rng.random((3, n)) - 0.5)
+    u[2] = 0
+    with capi.Context(cfg) as c:
+        c.upload_solid(solid)
+        got = []
+        for steps in ((3, 4, 6, 8, 1, 11), [1] * 33):
+            c.init_equilibrium(rho, u)
+            for s in steps:
+                c.step(s)
+            got.append(c.populations(np.float64))
+    assert np.isfinite(got[0]).all()
+    assert np.array_equal(*got)
