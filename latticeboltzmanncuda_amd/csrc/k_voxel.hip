@@ -13,7 +13,7 @@
 // A mesh whose faces close (every edge is run through as often one way as
 // the other) has a whole W at every node off its faces: the signed count of
 // the faces that a ray from the node crosses.  k_voxelize_lines counts them
-// along z, one wavefront per lattice line, with exact predicates, so that
+// along z, one wavefront per lattice line, the side of each edge exact, so that
 // the count is the W that the solid angles round to.  Other meshes take the
 // sum of solid angles (k_voxelize; same formulas as the host, double
 // precision, no contraction; only atan2 comes from the GPU's math library,
@@ -145,12 +145,15 @@ __global__ void __launch_bounds__(kBlock)
   boxes[f] = {{lo[0] - m, lo[1] - m, lo[2] - m}, {hi[0] + m, hi[1] + m, hi[2] + m}};
 }
 
-// Sign of a x b (two components), exact for the doubles given: where the
-// rounded products are equal their rounding errors decide.
+// Sign of a x b (two components), exact for the doubles given (without
+// overflow and underflow, which float coordinates do not reach): rounding
+// keeps the order, so products that round apart lie so, and where they round
+// alike their rounding errors, which fma gives exactly, decide.
 __device__ __forceinline__ int cross_sign(double ax, double ay, double bx, double by) {
   const double p = ax * by, q = ay * bx;
-  const double d = (p - q) + (fma(ax, by, -p) - fma(ay, bx, -q));
-  return d > 0.0 ? 1 : (d < 0.0 ? -1 : 0);
+  if (p != q) return p > q ? 1 : -1;
+  const double e = fma(ax, by, -p), f = fma(ay, bx, -q);
+  return e > f ? 1 : (e < f ? -1 : 0);
 }
 
 // Side of the edge a -> b on which the origin's projection lies, a and b
