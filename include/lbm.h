@@ -208,9 +208,10 @@ int lbm_set_force(lbm_ctx* ctx, const float in[3]);
 int lbm_get_force(lbm_ctx* ctx, float out[3]);
 
 /* ------------------------------------------------------------ stepping */
-/* n fused steps.  Standard mode: BGK pull collide+stream (D2Q9 lattices
- * take up to eight steps in one launch, large D3Q19 lattices in FP32 or FP64
- * two; as many launches, odd or even, as steps; one step of a D2Q9 lattice
+/* n fused steps.  Standard mode: BGK pull collide+stream (where that is
+ * faster, D2Q9 lattices take up to eight steps in one launch and, from calls
+ * of four steps on, large D3Q19 lattices in FP32 or FP64 two; as many launches,
+ * odd or even, as steps: lbm_step_route; one step of a D2Q9 lattice
  * with 16-bit storage larger than the Infinity Cache updates 4 or 2 nodes per
  * thread; the environment variable LBM_GROUP_STEP=0 / 1 asks D2Q9 lattices
  * for one step at a time and turns the latter off / on for any size -- the

@@ -8,10 +8,11 @@
 //
 // The per-node update is std_node_step (lbm_step_node.h); large D2Q9
 // lattices with 16-bit storage take std_group_step instead, 2 or 4 nodes
-// per thread (k_std_stepv, chosen by group_step_width).  Several steps of a
-// D2Q9 lattice go in one launch: box by box in LDS for the small ones
-// (k_std_box), as a sweep for the large ones (k_std_sweep); two steps of a
-// large D3Q19 lattice go in one pass along x (k_std_march).  Lattices whose
+// per thread (k_std_stepv, chosen by group_step_width), small 3-D lattices
+// k_std_early.  Where it is faster (plan_steps), several steps of a D2Q9
+// lattice go in one launch: box by box in LDS for the small ones (k_std_box),
+// as a sweep for the large ones (k_std_sweep); two steps of a large D3Q19
+// lattice go in one pass along x (k_std_march).  Lattices whose
 // two population copies exceed the Infinity Cache use non-temporal stores
 // and walk the tiles in opposite orders on consecutive steps; smaller ones
 // use ordinary stores and a fixed order (both measured fastest on MI355X).
