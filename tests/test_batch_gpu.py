@@ -320,3 +320,23 @@ def test_short_chunks_of_several_types_cost_no_more_than_their_launches():
         b.close()
     for (cfg, solid), g in list(zip(specs, got))[::5]:
         assert np.array_equal(g, run_alone(cfg, solid, 20 + 5 * 20 * 20))
+
+
+def test_short_and_long_calls_in_turn_equal_alone():
+    # a call of 8 steps captures one graph of both types, one of 16 a graph
+    # per type, which the short calls after it take too
+    say("case: short and long calls in chunks of 8, two lattice types")
+    specs = [(capi.make_config(90, 80 + k, 1, lattice=9, tau=0.7, lid_face=3,
+                               lid_u=(0.05, 0, 0)), None) for k in range(2)]
+    specs += [(capi.make_config(28, 27, 28 + k, lattice=19, tau=0.7,
+                                periodic=(1, 0, 0), force=(1e-5, 0, 0)), None)
+              for k in range(2)]
+    calls = [8, 8, 16, 8, 35, 4, 800, 9]
+    with capi.Batch(capi.STORE_F32) as b:
+        ms = [b.add(*s) for s in specs]
+        for n in calls:
+            b.step(n, 8)
+        b.synchronize()
+        got = [m.populations() for m in ms]
+    for s, g in zip(specs, got):
+        assert np.array_equal(g, run_alone(*s, sum(calls)))
